@@ -324,8 +324,9 @@ int lscomp_error_stats_u16(const uint16_t *d_orig, const uint16_t *d_dec, size_t
  * over the windows.  Window moments are exact (the reference rounds two-pass
  * double sums), so results agree to about 1e-12 relative.  Where the
  * reference prints an error and returns 0/0 (a dimension below 7), this
- * returns LSCOMP_ERR_INVALID_ARG.  Synchronous on `stream`; allocates one
- * double per workgroup. */
+ * returns LSCOMP_ERR_INVALID_ARG.  Synchronous on `stream`; the partial sums
+ * live in the stream's scratch area (or, above 1 MiB, in a temporary
+ * allocation). */
 int lscomp_ssim_u16(const uint16_t *d_orig, const uint16_t *d_dec, lscomp_dim3 dims, double *ssim,
                     hipStream_t stream);
 

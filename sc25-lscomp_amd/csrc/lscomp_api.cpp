@@ -171,8 +171,10 @@ struct Scratch {
     uint64_t *tile_off = nullptr;  // device, cap_tiles + 1 decode tile offsets
     uint64_t launches = 0;         // epochs used since the status words were cleared
     Ctrl *host = nullptr;          // pinned readback of ctrl
+    void *aux = nullptr;           // device, kAuxKeep bytes (AuxLease), allocated at first use
     std::mutex mu;
 };
+static_assert(sizeof(Ctrl) >= 256 + kAuxHost, "the host readback area holds a Ctrl head and an AuxLease result");
 
 std::mutex g_mu;
 std::map<std::pair<int, hipStream_t>, Scratch *> g_scratch;
@@ -267,6 +269,36 @@ int take_errors(Scratch *s)
 }  // namespace
 
 namespace lsc {
+
+AuxLease::AuxLease(hipStream_t stream, size_t bytes, size_t host_bytes) : stream_(stream)
+{
+    Scratch *s = get_scratch(stream);
+    if (!s || host_bytes > kAuxHost) {
+        st_ = LSCOMP_ERR_HIP;
+        return;
+    }
+    lk_ = std::unique_lock<std::mutex>(s->mu);
+    host_ = (uint8_t *)s->host + 256;   // beside the control head's readback
+    if (bytes > kAuxKeep) {
+        st_ = hip_fail(hipMalloc(&dev_, bytes), "hipMalloc");
+        own_ = st_ == LSCOMP_OK;
+        return;
+    }
+    if (!s->aux) st_ = hip_fail(hipMalloc(&s->aux, kAuxKeep), "hipMalloc");
+    dev_ = s->aux;
+}
+
+AuxLease::~AuxLease()
+{
+    if (own_) (void)hipFree(dev_);
+}
+
+int AuxLease::read_back(size_t bytes)
+{
+    int st = hip_fail(hipMemcpyAsync(host_, dev_, bytes, hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync");
+    if (st) return st;
+    return hip_fail(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+}
 
 // Validates a compression call and fills its Item (no HIP calls).
 int prepare_compress(const uint16_t *d_in, uint8_t *d_out, size_t cap, lscomp_dim3 dims, lscomp_bins4 bins,
@@ -585,6 +617,7 @@ void lscomp_release_all(void)
         if (s->tile_off) (void)hipFree(s->tile_off);
         if (s->ctrl) (void)hipFree(s->ctrl);
         if (s->host) (void)hipHostFree(s->host);
+        if (s->aux) (void)hipFree(s->aux);
         delete s;
         itr = g_scratch.erase(itr);
     }

@@ -3,6 +3,7 @@
 #pragma once
 #include <atomic>
 #include <functional>
+#include <mutex>
 #include <vector>
 #include <stdint.h>
 
@@ -44,6 +45,32 @@ int prepare_compress(const uint16_t *d_in, uint8_t *d_out, size_t cap, lscomp_di
                      float p, uint32_t tile, Item &it);
 int prepare_decompress(uint16_t *d_out, const uint8_t *d_in, size_t in_bytes, lscomp_dim3 dims,
                        lscomp_bins4 bins, uint32_t tile, Item &it);
+// Device memory for a synchronous call's partial results, and pinned host
+// memory to read a result of up to `host_bytes` (at most kAuxHost) back: the
+// (device, stream) scratch area's while the lease lives (its lock is held; up
+// to kAuxKeep bytes stay allocated until lscomp_release_all), a temporary
+// allocation above that.
+constexpr size_t kAuxKeep = 1u << 20, kAuxHost = 1024;
+class AuxLease {
+public:
+    AuxLease(hipStream_t stream, size_t bytes, size_t host_bytes);
+    ~AuxLease();
+    AuxLease(const AuxLease &) = delete;
+    AuxLease &operator=(const AuxLease &) = delete;
+    int status() const { return st_; }
+    void *device() const { return dev_; }
+    const void *host() const { return host_; }
+    // copies the first `bytes` of the device memory to host() and waits for the stream
+    int read_back(size_t bytes);
+
+private:
+    std::unique_lock<std::mutex> lk_;
+    hipStream_t stream_;
+    void *dev_ = nullptr, *host_ = nullptr;
+    bool own_ = false;
+    int st_ = LSCOMP_OK;
+};
+
 // Look-back words carry a 26-bit epoch: cleared at least every 2^25 launches
 // that use them, no stale word of an equal epoch survives.
 constexpr uint64_t kEpochClearPeriod = 1ull << 25;

@@ -5,7 +5,7 @@
 // - 10 log10(mse), normErr = sqrt(sum err^2), normErr_norm = normErr /
 // sqrt(sum dec^2), nrmse = sqrt(mse)/range; plus the maximum absolute error
 // and the maximum pointwise relative error over nonzero originals.  Sums are
-// exact 64-bit integers (uint16 data), reduced per wave and then atomically.
+// exact 64-bit integers (uint16 data), one partial per workgroup.
 // One pass, HBM-bound: 4 bytes read per element pair.  Also the mean SSIM
 // of the reference's computeSSIM (cuLSZ_utility.cu:757-886), and the plain
 // copy used to measure copy bandwidth and to calibrate the HBM byte counters.
@@ -20,81 +20,142 @@
 
 namespace lsc {
 
+// 16 bytes at 4-byte alignment (global_load_dwordx4 takes dword alignment).
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), __aligned__(4)));
+
+__device__ __forceinline__ uint32_t pk_max(uint32_t a, uint32_t b)
+{
+    return as_u32(__builtin_elementwise_max(as_u16x2(a), as_u16x2(b)));
+}
+__device__ __forceinline__ uint32_t pk_min(uint32_t a, uint32_t b)
+{
+    return as_u32(__builtin_elementwise_min(as_u16x2(a), as_u16x2(b)));
+}
+__device__ __forceinline__ uint32_t pk_sub(uint32_t a, uint32_t b) { return as_u32(as_u16x2(a) - as_u16x2(b)); }
+
+constexpr uint32_t kMetricWg = 512, kMetricGrid = 1024;   // threads per workgroup, workgroups at most
+
+// Sums and extrema of one thread, one workgroup or the whole pair of volumes.
+// The largest relative error is kept as the fraction rel_e / rel_a: rounding is
+// monotone, so the largest rounded quotient is the rounded largest quotient,
+// and two fractions of 16-bit values compare exactly by 32-bit products.
 struct MetricAcc {
     unsigned long long sum_sq_err, sum_sq_dec;
-    uint32_t max_err, min_orig, max_orig, max_rel_bits;   // max_rel as float bits (non-negative)
+    uint32_t max_err, min_orig, max_orig;
+    uint32_t rel_e, rel_a, pad;
+
+    __device__ __forceinline__ void rel(uint32_t e, uint32_t a)
+    {
+        e = a ? e : 0u;
+        if (e * rel_a > rel_e * a) {
+            rel_e = e;
+            rel_a = a;
+        }
+    }
+    __device__ __forceinline__ void pair(uint32_t a, uint32_t d)
+    {
+        const uint32_t e = a > d ? a - d : d - a;
+        sum_sq_err += (uint64_t)e * e;
+        sum_sq_dec += (uint64_t)d * d;
+        max_err = e > max_err ? e : max_err;
+        min_orig = a < min_orig ? a : min_orig;
+        max_orig = a > max_orig ? a : max_orig;
+        rel(e, a);
+    }
+    __device__ __forceinline__ void merge(const MetricAcc &o)
+    {
+        sum_sq_err += o.sum_sq_err;
+        sum_sq_dec += o.sum_sq_dec;
+        max_err = o.max_err > max_err ? o.max_err : max_err;
+        min_orig = o.min_orig < min_orig ? o.min_orig : min_orig;
+        max_orig = o.max_orig > max_orig ? o.max_orig : max_orig;
+        rel(o.rel_e, o.rel_a);
+    }
 };
 
-__global__ void metrics_init_kernel(MetricAcc *acc)
+__device__ __forceinline__ MetricAcc metric_zero() { return MetricAcc{0, 0, 0, 0xffffu, 0, 0, 1, 0}; }
+
+// Merge over the workgroup's WG threads; thread 0 holds the result.
+template <uint32_t WG>
+__device__ __forceinline__ void metric_reduce(MetricAcc &m)
 {
-    acc->sum_sq_err = 0;
-    acc->sum_sq_dec = 0;
-    acc->max_err = 0;
-    acc->min_orig = 0xffffu;
-    acc->max_orig = 0;
-    acc->max_rel_bits = 0;
+    __shared__ MetricAcc part[WG / 64];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1)
+        m.merge(MetricAcc{__shfl_xor(m.sum_sq_err, o, 64), __shfl_xor(m.sum_sq_dec, o, 64), __shfl_xor(m.max_err, o, 64),
+                          __shfl_xor(m.min_orig, o, 64), __shfl_xor(m.max_orig, o, 64), __shfl_xor(m.rel_e, o, 64),
+                          __shfl_xor(m.rel_a, o, 64), 0});
+    if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (uint32_t w = 1; w < WG / 64; w++) m.merge(part[w]);
 }
 
-__device__ __forceinline__ void acc_pair(uint32_t a, uint32_t d, uint64_t &se, uint64_t &sd, uint32_t &me,
-                                         uint32_t &mn, uint32_t &mx, float &mr)
+// One pass over both volumes, read-bound: 16-byte loads of `n8` groups of 8
+// elements starting at element `head` (both volumes dword aligned there), the
+// elements before and after one by one.  A group's arithmetic is on packed
+// pairs (absolute difference, extrema, dot products for the squares: their sum
+// over 8 elements fits 32 bits while all are below 2^14, otherwise element by
+// element).  Each workgroup writes one partial (metrics_finish_kernel merges
+// them): six 64- and 32-bit atomics per wave on one line cost 2.37 ms at 512 x
+// 1024 x 1024, whatever the size above some thousand waves, against 0.37 ms.
+__global__ __launch_bounds__(kMetricWg) void metrics_kernel(const uint16_t *__restrict__ orig,
+                                                            const uint16_t *__restrict__ dec, uint64_t n,
+                                                            uint32_t head, uint64_t n8, MetricAcc *__restrict__ part)
 {
-    const uint32_t e = a > d ? a - d : d - a;
-    se += (uint64_t)e * e;
-    sd += (uint64_t)d * d;
-    me = e > me ? e : me;
-    mn = a < mn ? a : mn;
-    mx = a > mx ? a : mx;
-    if (a) {
-        const float r = (float)e / (float)a;
-        mr = r > mr ? r : mr;
-    }
-}
-
-__global__ __launch_bounds__(256) void metrics_kernel(const uint16_t *__restrict__ orig,
-                                                      const uint16_t *__restrict__ dec, uint64_t n,
-                                                      MetricAcc *acc)
-{
-    uint64_t se = 0, sd = 0;
-    uint32_t me = 0, mn = 0xffffu, mx = 0;
-    float mr = 0.0f;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    const uint64_t n8 = n / 8;
-    const bool vec = (((uintptr_t)orig | (uintptr_t)dec) & 15) == 0;
-    uint64_t tail = 0;
-    if (vec) {
-        for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n8; i += stride) {
-            const uint4 a = ((const uint4 *)orig)[i], d = ((const uint4 *)dec)[i];
-            const uint32_t av[4] = {a.x, a.y, a.z, a.w}, dv[4] = {d.x, d.y, d.z, d.w};
+    MetricAcc m = metric_zero();
+    const uint64_t stride = (uint64_t)gridDim.x * kMetricWg, first = (uint64_t)blockIdx.x * kMetricWg + threadIdx.x;
+    const u32x4_a4 *va = (const u32x4_a4 *)(orig + head), *vd = (const u32x4_a4 *)(dec + head);
+    uint32_t mn2 = 0xffffffffu, mx2 = 0, me2 = 0;   // packed extrema
+    for (uint64_t i = first; i < n8; i += stride) {
+        const u32x4_a4 a = va[i], d = vd[i];
+        uint32_t e[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            mn2 = pk_min(mn2, a[k]);
+            mx2 = pk_max(mx2, a[k]);
+            e[k] = pk_sub(pk_max(a[k], d[k]), pk_min(a[k], d[k]));
+            me2 = pk_max(me2, e[k]);
+            m.rel(e[k] & 0xffffu, a[k] & 0xffffu);
+            m.rel(e[k] >> 16, a[k] >> 16);
+        }
+        if (((e[0] | e[1] | e[2] | e[3] | d[0] | d[1] | d[2] | d[3]) & 0xc000c000u) == 0) {
+            uint32_t se = 0, sd = 0;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                acc_pair(av[k] & 0xffffu, dv[k] & 0xffffu, se, sd, me, mn, mx, mr);
-                acc_pair(av[k] >> 16, dv[k] >> 16, se, sd, me, mn, mx, mr);
+                se = dot2(e[k], e[k], se);
+                sd = dot2(d[k], d[k], sd);
+            }
+            m.sum_sq_err += se;
+            m.sum_sq_dec += sd;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint32_t e0 = e[k] & 0xffffu, e1 = e[k] >> 16, d0 = d[k] & 0xffffu, d1 = d[k] >> 16;
+                m.sum_sq_err += (uint64_t)(e0 * e0) + (uint64_t)(e1 * e1);
+                m.sum_sq_dec += (uint64_t)(d0 * d0) + (uint64_t)(d1 * d1);
             }
         }
-        tail = n8 * 8;
     }
-    for (uint64_t i = tail + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-        acc_pair(orig[i], dec[i], se, sd, me, mn, mx, mr);
-    // wave reduction, then one atomic per wave
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        se += __shfl_xor(se, o, 64);
-        sd += __shfl_xor(sd, o, 64);
-        const uint32_t me2 = __shfl_xor(me, o, 64), mn2 = __shfl_xor(mn, o, 64), mx2 = __shfl_xor(mx, o, 64);
-        const float mr2 = __shfl_xor(mr, o, 64);
-        me = me2 > me ? me2 : me;
-        mn = mn2 < mn ? mn2 : mn;
-        mx = mx2 > mx ? mx2 : mx;
-        mr = mr2 > mr ? mr2 : mr;
+    m.max_err = me2 >> 16 > (me2 & 0xffffu) ? me2 >> 16 : me2 & 0xffffu;
+    m.max_orig = mx2 >> 16 > (mx2 & 0xffffu) ? mx2 >> 16 : mx2 & 0xffffu;
+    m.min_orig = mn2 >> 16 < (mn2 & 0xffffu) ? mn2 >> 16 : mn2 & 0xffffu;
+    // the elements before the first group and after the last one
+    const uint64_t rest = n - 8 * n8;
+    for (uint64_t i = first; i < rest; i += stride) {
+        const uint64_t at = i < head ? i : i + 8 * n8;
+        m.pair(orig[at], dec[at]);
     }
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&acc->sum_sq_err, (unsigned long long)se);
-        atomicAdd(&acc->sum_sq_dec, (unsigned long long)sd);
-        atomicMax(&acc->max_err, me);
-        atomicMin(&acc->min_orig, mn);
-        atomicMax(&acc->max_orig, mx);
-        atomicMax(&acc->max_rel_bits, __float_as_uint(mr));   // non-negative floats order like their bits
-    }
+    metric_reduce<kMetricWg>(m);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
+}
+
+__global__ __launch_bounds__(kMetricGrid) void metrics_finish_kernel(const MetricAcc *__restrict__ part, uint32_t np,
+                                                                     MetricAcc *__restrict__ out)
+{
+    MetricAcc m = threadIdx.x < np ? part[threadIdx.x] : metric_zero();
+    metric_reduce<kMetricGrid>(m);
+    if (threadIdx.x == 0) *out = m;
 }
 
 // Plain copy: each workgroup copies one contiguous 16 KiB chunk, four 16-byte
@@ -124,160 +185,263 @@ __global__ void copy_tail_kernel(uint8_t *dst, const uint8_t *src, uint32_t n)
 // when R = 0) and c3 = c2 / 2.
 //
 // Separable window sums instead of the reference's two passes over every
-// window's 343 points.  A workgroup owns 64 x 4 windows along (size0, size1)
-// and up to 64 windows along size2, and walks that slab plane by plane: each
-// plane's 13 x 133 patch of both volumes goes to LDS; row sums over 7 columns
-// (at column stride 2) for 13 rows x 64 windows; each thread sums 7 rows of
-// its window into the plane's moments P; along size2 a window is the sum of
-// three plane pairs and one plane (planes 2k .. 2k+6), kept in registers.
-// Moments are exact: integer sums of values, double sums of squares and
-// products (integers below 2^53), so the variances and the covariance are
-// n*S_xx - S_x^2 (exact 64-bit integers) over n^2, correctly rounded, where the
-// reference rounds a two-pass double sum.  Each workgroup writes one partial
-// sum, reduced in a fixed order; the host adds the partials in order, so the
-// result does not depend on scheduling.
+// window's 343 points, and the product of the three terms in closed form:
+// with c3 = c2 / 2, contrast * structure = (2 cov + c2) / (var_x + var_y + c2)
+// (the standard deviations cancel), so a window needs its sums of x, y, xy and
+// x^2 + y^2, the original's extrema and one division.  All sums are exact
+// integers, and n^2 times each factor's numerator and denominator (n = 343) is
+// formed from them in doubles, where the reference rounds a two-pass double
+// sum.
+//
+// ALU-bound, so the mapping is chosen for few operations per window.  A lane
+// owns one window column along size0 and kSsimJ windows along size1, and walks
+// planes (size2).  Per row it loads its 8 elements (16 bytes at a dword
+// boundary; neighbouring lanes overlap in L1) and forms the 7-element sums by
+// packed dot products in 32 bits; a plane with a value of 2^14 or more in any
+// of a lane's rows is formed again by 64-bit products.  Along size1, and then
+// along size2, windows overlap by 5 of 7, so a window is the sum of three
+// disjoint pairs and one row (plane); pairs stay in registers, nothing goes
+// through LDS and there is no barrier in the loop.  512 x 1024 x 1024: 1.23 ms
+// against 3.19 ms with one window per thread, double sums through LDS, square
+// roots, divisions and three barriers per plane.  Two windows per lane run at
+// 3 waves per SIMD; with 3 or 4 a plane costs fewer row sums per window but
+// the sums held along size2 leave 2 waves (1.33 and 1.93 ms).
+//
+// Each workgroup writes one partial sum, reduced in a fixed order (here and in
+// ssim_finish_kernel), so the result does not depend on scheduling.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kSsimT0 = 64, kSsimT1 = 4, kSsimChunk = 64;   // windows per workgroup along size0, size1, size2
-constexpr uint32_t kSsimPC = 2 * kSsimT0 + 5, kSsimPR = 2 * kSsimT1 + 5;   // patch columns (133) and rows (13)
-constexpr uint32_t kSsimPitch = 136;                                       // u16 per patch row (even, >= 134)
+constexpr uint32_t kSsimJ = 2;                            // windows of a lane along size1
+constexpr uint32_t kSsimT0 = 64, kSsimT1 = 4 * kSsimJ;    // windows of a workgroup (4 waves) along size0, size1
+constexpr uint32_t kSsimRows = 2 * kSsimJ + 5;            // rows of a lane's windows
 
+// Sums over 7 elements of one row; extrema still in two halves.
+struct SsimRow {
+    uint32_t sx, sy, mx2, mn2;
+    uint64_t sxy, sqq;   // sums of x y and of x^2 + y^2
+};
+// Sums over a 7 x 7 patch of a plane, and over planes; mm = max | (65535 - min) << 16.
 struct SsimMom {
-    uint32_t sx, sy, mn, mx;   // sums of both volumes, min and max of the original
-    double sxx, syy, sxy;      // exact integer sums
+    uint32_t sx, sy, mm;
+    uint64_t sxy, sqq;
 };
 
+__device__ __forceinline__ SsimRow row_add(const SsimRow &a, const SsimRow &b)
+{
+    return {a.sx + b.sx, a.sy + b.sy, pk_max(a.mx2, b.mx2), pk_min(a.mn2, b.mn2), a.sxy + b.sxy, a.sqq + b.sqq};
+}
 __device__ __forceinline__ SsimMom mom_add(const SsimMom &a, const SsimMom &b)
 {
-    return {a.sx + b.sx, a.sy + b.sy, a.mn < b.mn ? a.mn : b.mn, a.mx > b.mx ? a.mx : b.mx,
-            a.sxx + b.sxx, a.syy + b.syy, a.sxy + b.sxy};
+    return {a.sx + b.sx, a.sy + b.sy, pk_max(a.mm, b.mm), a.sxy + b.sxy, a.sqq + b.sqq};
+}
+__device__ __forceinline__ SsimMom mom_of(const SsimRow &r)
+{
+    const uint32_t mx = pk_max(r.mx2, r.mx2 >> 16) & 0xffffu, mn = pk_min(r.mn2, r.mn2 >> 16 | 0xffff0000u) & 0xffffu;
+    return {r.sx, r.sy, mx | (0xffffu - mn) << 16, r.sxy, r.sqq};
 }
 
-__device__ double ssim_of(const SsimMom &m)
+__device__ __forceinline__ double ssim_of(const SsimMom &m)
 {
 #pragma clang fp contract(off)
-    const double np = 343.0;
-    const double x_mean = (double)m.sx / np, y_mean = (double)m.sy / np;
-    const int64_t sx = m.sx, sy = m.sy;
-    const double n2 = np * np;
-    const double var_x = (double)(343 * (int64_t)m.sxx - sx * sx) / n2;
-    const double var_y = (double)(343 * (int64_t)m.syy - sy * sy) / n2;
-    const double cov = (double)(343 * (int64_t)m.sxy - sx * sy) / n2;
-    const double x_sigma = sqrt(var_x), y_sigma = sqrt(var_y);
-    const float range = (float)(m.mx - m.mn);
-    double c1, c2;
-    if (range == 0.0f) {
-        c1 = 0.01 * 0.01;
-        c2 = 0.03 * 0.03;
-    } else {
-        c1 = 0.01 * 0.01 * range * range;
-        c2 = 0.03 * 0.03 * range * range;
-    }
-    const double c3 = c2 / 2;
-    const double luminance = (2 * x_mean * y_mean + c1) / (x_mean * x_mean + y_mean * y_mean + c1);
-    const double contrast = (2 * x_sigma * y_sigma + c2) / (x_sigma * x_sigma + y_sigma * y_sigma + c2);
-    const double structure = (cov + c3) / (x_sigma * y_sigma + c3);
-    return luminance * contrast * structure;
+    const double n = 343.0, n2 = n * n;
+    const double sx = (double)m.sx, sy = (double)m.sy;
+    const double range = (double)((m.mm & 0xffffu) - (0xffffu - (m.mm >> 16)));
+    const double r2 = range == 0.0 ? 1.0 : range * range;
+    const double c1 = 0.01 * 0.01 * n2 * r2, c2 = 0.03 * 0.03 * n2 * r2;
+    // integers below 2^51: exact in doubles
+    const double pxy = sx * sy, pqq = sx * sx + sy * sy;
+    const double cov = n * (double)m.sxy - pxy, var = n * (double)m.sqq - pqq;
+    return ((2.0 * pxy + c1) * (2.0 * cov + c2)) / ((pqq + c1) * (var + c2));
 }
 
-// One workgroup per (size0 tile, size1 tile, size2 chunk) of windows; grid
-// nb0 * nb1 * nchunks workgroups of 256 threads; partial[blockIdx.x] = the
-// sum of the SSIM of its windows.
-__global__ __launch_bounds__(256) void ssim_kernel(const uint16_t *__restrict__ ori, const uint16_t *__restrict__ dec,
-                                                   uint32_t X, uint32_t Y, uint32_t Z, uint32_t n0, uint32_t n1,
-                                                   uint32_t n2, uint32_t nb0, uint32_t nb1, double *partial)
+// The 7 elements of a lane's row as 4 words: 16 bytes from the dword boundary
+// at or before the first element.  `odd` (uniform): the row's first element is
+// the word's upper half and the last word is whole; else the last word's upper
+// half is an eighth element that does not count.
+template <bool kWide>
+__device__ __forceinline__ SsimRow ssim_row(u32x4_a4 x, u32x4_a4 y, bool odd, uint32_t &seen)
 {
-    __shared__ __align__(16) uint16_t xs[kSsimPR][kSsimPitch], ys[kSsimPR][kSsimPitch];
-    __shared__ uint32_t r_sx[kSsimPR][kSsimT0], r_sy[kSsimPR][kSsimT0], r_mn[kSsimPR][kSsimT0],
-        r_mx[kSsimPR][kSsimT0];
-    __shared__ double r_sxx[kSsimPR][kSsimT0], r_syy[kSsimPR][kSsimT0], r_sxy[kSsimPR][kSsimT0];
+    const uint32_t m0 = odd ? 0xffff0000u : 0xffffffffu, m3 = odd ? 0xffffffffu : 0xffffu;
+    const uint32_t lo = x[0] | ~m0, hi = x[3] | ~m3;   // for the minimum
+    x[0] &= m0;
+    y[0] &= m0;
+    x[3] &= m3;
+    y[3] &= m3;
+    SsimRow r;
+    r.mx2 = pk_max(pk_max(x[0], x[1]), pk_max(x[2], x[3]));
+    r.mn2 = pk_min(pk_min(lo, x[1]), pk_min(x[2], hi));
+    r.sx = 0;
+    r.sy = 0;
+    uint32_t xy = 0, qq = 0;
+    r.sxy = 0;
+    r.sqq = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        r.sx = dot2(x[k], 0x00010001u, r.sx);
+        r.sy = dot2(y[k], 0x00010001u, r.sy);
+        if (kWide) {
+            const uint32_t x0 = x[k] & 0xffffu, x1 = x[k] >> 16, y0 = y[k] & 0xffffu, y1 = y[k] >> 16;
+            r.sxy += (uint64_t)(x0 * y0) + (uint64_t)(x1 * y1);
+            r.sqq += (uint64_t)(x0 * x0) + (uint64_t)(x1 * x1) + (uint64_t)(y0 * y0) + (uint64_t)(y1 * y1);
+        } else {   // 14 products below 2^28: 32 bits hold their sum
+            xy = dot2(x[k], y[k], xy);
+            qq = dot2(x[k], x[k], qq);
+            qq = dot2(y[k], y[k], qq);
+        }
+    }
+    if (!kWide) {
+        seen |= x[0] | x[1] | x[2] | x[3] | y[0] | y[1] | y[2] | y[3];
+        r.sxy = xy;
+        r.sqq = qq;
+    }
+    return r;
+}
+
+// The 16 bytes of a row by elements, without the one that belongs to no window.
+__device__ __forceinline__ u32x4_a4 ssim_elements(const uint16_t *q, bool odd)
+{
+    uint32_t w0 = 0, w1 = 0, w2 = 0, w3 = 0;
+#pragma unroll 1
+    for (uint32_t k = 0; k < 8; k++) {   // shifted in from above
+        const uint32_t e = (odd ? k != 0 : k != 7) ? q[k] : 0u;
+        w0 = __builtin_amdgcn_alignbit(w1, w0, 16);
+        w1 = __builtin_amdgcn_alignbit(w2, w1, 16);
+        w2 = __builtin_amdgcn_alignbit(w3, w2, 16);
+        w3 = w3 >> 16 | e << 16;
+    }
+    return u32x4_a4{w0, w1, w2, w3};
+}
+
+// The plane sums of a lane's kSsimJ windows: P[j] over rows 2j .. 2j + 6 of the
+// kSsimRows rows from row y0 of the plane that starts at element `plane` (rows
+// past the volume repeat its last one; their windows are not counted).
+// kAny: 64-bit products, and rows by elements when `elements` is set; else
+// 32-bit ones, and the bits seen in any value are returned.
+template <bool kAny>
+__device__ __forceinline__ uint32_t ssim_plane(const uint16_t *ori, const uint16_t *dec, uint64_t plane, uint32_t Y,
+                                               uint32_t Z, uint32_t y0, uint32_t c, uint32_t odd0, bool elements,
+                                               SsimMom P[kSsimJ])
+{
+    SsimRow even{}, a0{}, a1{}, a2{};   // the last even row, the last three pairs
+    uint32_t seen = 0;
+    const auto step = [&](uint32_t r) -> SsimMom {
+        const uint64_t row = plane + (uint64_t)(y0 + r < Y ? y0 + r : Y - 1u) * Z;
+        const bool odd = (((uint32_t)row ^ odd0) & 1u) != 0;
+        const uint16_t *qx = ori + (row + c - odd), *qy = dec + (row + c - odd);
+        u32x4_a4 x, y;
+        if (kAny && elements) {
+            x = ssim_elements(qx, odd);
+            y = ssim_elements(qy, odd);
+        } else {
+            x = *(const u32x4_a4 *)qx;
+            y = *(const u32x4_a4 *)qy;
+        }
+        const SsimRow v = ssim_row<kAny>(x, y, odd, seen);
+        if (r & 1u) {
+            a0 = a1;
+            a1 = a2;
+            a2 = row_add(even, v);
+            return {};
+        }
+        even = v;
+        return mom_of(row_add(row_add(a0, a1), row_add(a2, v)));
+    };
+    if (kAny) {   // rare: a rolled loop, so that the kernel holds the row's code only once more
+#pragma unroll 1
+        for (uint32_t r = 0; r < kSsimRows; r++) {
+            const SsimMom m = step(r);
+#pragma unroll
+            for (uint32_t j = 0; j < kSsimJ; j++)
+                if (r == 2u * j + 6u) P[j] = m;
+        }
+    } else {
+#pragma unroll
+        for (uint32_t r = 0; r < kSsimRows; r++) {
+            const SsimMom m = step(r);
+            if (r >= 6u && (r & 1u) == 0) P[(r - 6u) / 2u] = m;
+        }
+    }
+    return seen;
+}
+
+// One workgroup per (size0 tile, size1 tile, size2 chunk) of windows; grid nb0
+// * nb1 * nchunks workgroups of 256 threads; partial[blockIdx.x] = the sum of
+// the SSIM of its windows.  odd0: bit 0 (1) is set when the original (decoded)
+// volume starts at 2 mod 4.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void ssim_kernel(
+    const uint16_t *__restrict__ ori, const uint16_t *__restrict__ dec, uint32_t X, uint32_t Y, uint32_t Z, uint32_t n0,
+    uint32_t n1, uint32_t n2, uint32_t nb0, uint32_t nb1, uint32_t chunk, uint32_t odd0, double *__restrict__ partial)
+{
     __shared__ double wsum[4];
-    const uint32_t tid = threadIdx.x, t0 = tid & 63u, t1 = tid >> 6;
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint32_t blk = blockIdx.x;
     const uint32_t b0 = blk % nb0;
     blk /= nb0;
-    const uint32_t b1 = blk % nb1, c2 = blk / nb1;
-    const uint32_t o0b = b0 * kSsimT0, o1b = b1 * kSsimT1, o2b = c2 * kSsimChunk;
-    const uint32_t o2e = o2b + kSsimChunk < n2 ? o2b + kSsimChunk : n2;
-    const uint64_t col0 = 2ull * o0b, row0 = 2ull * o1b;
-    const bool mine = o0b + t0 < n0 && o1b + t1 < n1;
-    // planes [2 o2b, 2 (o2e - 1) + 7): the last is at most X - 1 since o2e <= n2
-    const uint32_t pb = 2u * o2b, pe = 2u * (o2e - 1u) + 7u;
-    (void)X;
-
-    SsimMom q0{}, q1{}, q2{}, pev{};   // the last three plane pairs, the last even plane
+    const uint32_t b1 = blk % nb1, b2 = blk / nb1;
+    const uint32_t o0 = b0 * kSsimT0 + lane, o1 = b1 * kSsimT1 + wave * kSsimJ, o2 = b2 * chunk;
+    const uint32_t nw = n2 - o2 < chunk ? n2 - o2 : chunk;   // windows along size2
+    const uint32_t c = 2u * (o0 < n0 ? o0 : n0 - 1u);        // first element of the window's rows
+    const bool mixed = odd0 == 1u || odd0 == 2u;             // the volumes' rows differ in alignment
     double acc = 0.0;
-    for (uint32_t p = pb; p < pe; p++) {
-        // 1. the plane's patch (zeros outside the volume: only windows that
-        //    are not counted read them)
-        for (uint32_t e = tid; e < kSsimPR * kSsimPC; e += 256u) {
-            const uint32_t r = e / kSsimPC, c = e - r * kSsimPC;
-            const uint64_t gy = row0 + r, gz = col0 + c;
-            uint16_t a = 0, b = 0;
-            if (gy < Y && gz < Z) {
-                const uint64_t i = ((uint64_t)p * Y + gy) * Z + gz;
-                a = ori[i];
-                b = dec[i];
-            }
-            xs[r][c] = a;
-            ys[r][c] = b;
-        }
-        __syncthreads();
-        // 2. row sums: 7 columns from column 2w, read as four aligned pairs
-        for (uint32_t e = tid; e < kSsimPR * kSsimT0; e += 256u) {
-            const uint32_t r = e >> 6, w = e & 63u;
-            const uint32_t *xr = (const uint32_t *)&xs[r][0] + w, *yr = (const uint32_t *)&ys[r][0] + w;
-            uint32_t sx = 0, sy = 0, mn = 0xffffu, mx = 0;
-            double sxx = 0, syy = 0, sxy = 0;
+    if (o1 < n1) {
+        // carry: after an odd plane the last three pairs of planes, after an
+        // even one that plane; the last two pairs, the last one
+        SsimMom carry[kSsimJ] = {}, s2[kSsimJ] = {}, s1[kSsimJ] = {};
+        const uint64_t per_plane = (uint64_t)Y * Z;
+        uint64_t plane = 2ull * o2 * per_plane;
+        // planes 2 o2 .. 2 o2 + 2 nw + 4, the last one at most X - 1
+        for (uint32_t i = 0; i < 2u * nw + 5u; i++, plane += per_plane) {
+            SsimMom P[kSsimJ];
+            // a row's 16 bytes can leave a volume, by one element, only in its
+            // first row (a base at 2 mod 4) and in its last
+            const bool elements = mixed || (plane == 0 && o1 == 0 && odd0) ||
+                                  (plane == (X - 1u) * per_plane && 2u * o1 + kSsimRows >= Y);
+            uint32_t seen = 0xffffffffu;
+            if (!elements) seen = ssim_plane<false>(ori, dec, plane, Y, Z, 2u * o1, c, odd0, false, P);
+            if (__ballot((seen & 0xc000c000u) != 0))
+                ssim_plane<true>(ori, dec, plane, Y, Z, 2u * o1, c, odd0, elements, P);
+            if (i & 1u) {
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint32_t xw = xr[k], yw = yr[k];
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    if (k == 3 && h == 1) break;   // 7 columns
-                    const uint32_t a = h ? xw >> 16 : xw & 0xffffu, b = h ? yw >> 16 : yw & 0xffffu;
-                    sx += a;
-                    sy += b;
-                    mn = a < mn ? a : mn;
-                    mx = a > mx ? a : mx;
-                    const double da = (double)a, db = (double)b;
-                    sxx = fma(da, da, sxx);
-                    syy = fma(db, db, syy);
-                    sxy = fma(da, db, sxy);
+                for (uint32_t j = 0; j < kSsimJ; j++) {
+                    const SsimMom t = mom_add(carry[j], P[j]);
+                    carry[j] = mom_add(s2[j], t);
+                    s2[j] = mom_add(s1[j], t);
+                    s1[j] = t;
                 }
-            }
-            r_sx[r][w] = sx;
-            r_sy[r][w] = sy;
-            r_mn[r][w] = mn;
-            r_mx[r][w] = mx;
-            r_sxx[r][w] = sxx;
-            r_syy[r][w] = syy;
-            r_sxy[r][w] = sxy;
-        }
-        __syncthreads();
-        // 3. this thread's window in the plane: rows 2 t1 .. 2 t1 + 6
-        SsimMom P{0, 0, 0xffffu, 0, 0.0, 0.0, 0.0};
+            } else {
+                if (i >= 6u) {
 #pragma unroll
-        for (uint32_t k = 0; k < 7; k++) {
-            const uint32_t r = 2u * t1 + k;
-            P = mom_add(P, SsimMom{r_sx[r][t0], r_sy[r][t0], r_mn[r][t0], r_mx[r][t0], r_sxx[r][t0], r_syy[r][t0],
-                                   r_sxy[r][t0]});
-        }
-        // 4. along size2: window k covers pairs k, k+1, k+2 and plane 2k + 6
-        const uint32_t j = p - pb;
-        if ((j & 1u) == 0) {
-            if (j >= 6 && mine) acc += ssim_of(mom_add(mom_add(q0, q1), mom_add(q2, P)));
-            pev = P;
-        } else {
-            q0 = q1;
-            q1 = q2;
-            q2 = mom_add(pev, P);
+                    for (uint32_t j = 0; j < kSsimJ; j++) {
+                        const double s = ssim_of(mom_add(carry[j], P[j]));
+                        acc += o0 < n0 && o1 + j < n1 ? s : 0.0;
+                    }
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < kSsimJ; j++) carry[j] = P[j];
+            }
         }
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
-    if ((tid & 63u) == 0) wsum[t1] = acc;
+    if (lane == 0) wsum[wave] = acc;
     __syncthreads();
-    if (tid == 0) partial[blockIdx.x] = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
+    if (threadIdx.x == 0) partial[blockIdx.x] = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
+}
+
+// The sum of np partials in a fixed order: thread t adds t, t + 1024, ...
+__global__ __launch_bounds__(1024) void ssim_finish_kernel(const double *__restrict__ partial, uint64_t np,
+                                                           double *__restrict__ out)
+{
+    __shared__ double wsum[16];
+    double acc = 0.0;
+    for (uint64_t i = threadIdx.x; i < np; i += 1024u) acc += partial[i];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    if ((threadIdx.x & 63u) == 0) wsum[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (uint32_t w = 1; w < 16; w++) acc += wsum[w];
+        *out = acc;
+    }
 }
 
 }  // namespace lsc
@@ -309,19 +473,25 @@ extern "C" int lscomp_error_stats_u16(const uint16_t *d_orig, const uint16_t *d_
     using namespace lsc;
     if (!d_orig || !d_dec || !out || n == 0 || (((uintptr_t)d_orig | (uintptr_t)d_dec) & 1))
         return LSCOMP_ERR_INVALID_ARG;
-    MetricAcc *acc = nullptr, host{};
-    int st = hip_fail(hipMalloc((void **)&acc, sizeof(MetricAcc)), "hipMalloc");
+    // the first element from which both volumes are dword aligned; volumes of
+    // different alignment mod 4 have none and are read by elements
+    const uint32_t oa = (uint32_t)((uintptr_t)d_orig >> 1) & 1u, od = (uint32_t)((uintptr_t)d_dec >> 1) & 1u;
+    const uint64_t n8 = oa == od && n > oa ? (n - oa) / 8 : 0;
+    const uint32_t head = n8 ? oa : 0u;
+    const uint64_t work = n8 ? n8 : n;
+    uint64_t blocks = (work + kMetricWg - 1) / kMetricWg;
+    if (blocks > kMetricGrid) blocks = kMetricGrid;
+    AuxLease aux(stream, (kMetricGrid + 1) * sizeof(MetricAcc), sizeof(MetricAcc));
+    int st = aux.status();
     if (st) return st;
-    hipLaunchKernelGGL(metrics_init_kernel, dim3(1), dim3(1), 0, stream, acc);
-    uint64_t blocks = (n / 8 + 255) / 256;
-    if (blocks > 8192) blocks = 8192;
-    if (blocks == 0) blocks = 1;
-    hipLaunchKernelGGL(metrics_kernel, dim3((uint32_t)blocks), dim3(256), 0, stream, d_orig, d_dec, (uint64_t)n, acc);
+    MetricAcc *acc = (MetricAcc *)aux.device();
+    hipLaunchKernelGGL(metrics_kernel, dim3((uint32_t)blocks), dim3(kMetricWg), 0, stream, d_orig, d_dec, (uint64_t)n,
+                       head, n8, acc + 1);
+    hipLaunchKernelGGL(metrics_finish_kernel, dim3(1), dim3(kMetricGrid), 0, stream, acc + 1, (uint32_t)blocks, acc);
     st = hip_fail(hipGetLastError(), "metrics launch");
-    if (!st) st = hip_fail(hipMemcpyAsync(&host, acc, sizeof host, hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
-    if (!st) st = hip_fail(hipStreamSynchronize(stream), "hipStreamSynchronize");
-    (void)hipFree(acc);
+    if (!st) st = aux.read_back(sizeof(MetricAcc));
     if (st) return st;
+    const MetricAcc host = *(const MetricAcc *)aux.host();
     std::memset(out, 0, sizeof *out);
     out->n = n;
     out->max_abs_err = host.max_err;
@@ -329,9 +499,7 @@ extern "C" int lscomp_error_stats_u16(const uint16_t *d_orig, const uint16_t *d_
     out->max_orig = host.max_orig;
     out->sum_sq_err = host.sum_sq_err;
     out->sum_sq_dec = host.sum_sq_dec;
-    float mr;
-    std::memcpy(&mr, &host.max_rel_bits, sizeof mr);
-    out->max_rel_err = mr;
+    out->max_rel_err = (float)host.rel_e / (float)host.rel_a;   // a float quotient, as the pointwise ones are defined
     out->mse = (double)host.sum_sq_err / (double)n;
     out->range = (double)host.max_orig - (double)host.min_orig;
     out->psnr = 20.0 * std::log10(out->range) - 10.0 * std::log10(out->mse);   // inf when lossless
@@ -349,24 +517,26 @@ extern "C" int lscomp_ssim_u16(const uint16_t *d_orig, const uint16_t *d_dec, ls
     if (dims.x < 7 || dims.y < 7 || dims.z < 7) return LSCOMP_ERR_INVALID_ARG;   // no window fits
     const uint32_t n0 = (dims.z - 7) / 2 + 1, n1 = (dims.y - 7) / 2 + 1, n2 = (dims.x - 7) / 2 + 1;
     const uint32_t nb0 = (n0 + kSsimT0 - 1) / kSsimT0, nb1 = (n1 + kSsimT1 - 1) / kSsimT1;
-    const uint32_t nc = (n2 + kSsimChunk - 1) / kSsimChunk;
+    // windows of a workgroup along size2: a chunk of k reads 2 k + 5 planes, so
+    // 32 where the volume gives enough workgroups (3 waves per SIMD run at
+    // once), fewer for small volumes
+    uint32_t chunk = 32;
+    while (chunk > 4 && (uint64_t)nb0 * nb1 * ((n2 + chunk - 1) / chunk) < 2048) chunk /= 2;
+    const uint32_t nc = (n2 + chunk - 1) / chunk;
     const uint64_t blocks = (uint64_t)nb0 * nb1 * nc;
     if (blocks > 0x7fffffffull) return LSCOMP_ERR_TOO_LARGE;
-    double *partial = nullptr;
-    int st = hip_fail(hipMalloc((void **)&partial, blocks * sizeof(double)), "hipMalloc");
+    AuxLease aux(stream, (blocks + 1) * sizeof(double), sizeof(double));
+    int st = aux.status();
     if (st) return st;
-    std::vector<double> host(blocks);
+    double *partial = (double *)aux.device();
+    const uint32_t odd0 = (uint32_t)((uintptr_t)d_orig >> 1 & 1u) | (uint32_t)((uintptr_t)d_dec >> 1 & 1u) << 1;
     hipLaunchKernelGGL(ssim_kernel, dim3((uint32_t)blocks), dim3(256), 0, stream, d_orig, d_dec, dims.x, dims.y,
-                       dims.z, n0, n1, n2, nb0, nb1, partial);
+                       dims.z, n0, n1, n2, nb0, nb1, chunk, odd0, partial + 1);
+    hipLaunchKernelGGL(ssim_finish_kernel, dim3(1), dim3(1024), 0, stream, partial + 1, blocks, partial);
     st = hip_fail(hipGetLastError(), "ssim launch");
-    if (!st)
-        st = hip_fail(hipMemcpyAsync(host.data(), partial, blocks * sizeof(double), hipMemcpyDeviceToHost, stream),
-                      "hipMemcpyAsync");
-    if (!st) st = hip_fail(hipStreamSynchronize(stream), "hipStreamSynchronize");
-    (void)hipFree(partial);
+    if (!st) st = aux.read_back(sizeof(double));
     if (st) return st;
-    double sum = 0.0;
-    for (double v : host) sum += v;
+    const double sum = *(const double *)aux.host();
     *ssim = sum / ((double)n0 * (double)n1 * (double)n2);
     return LSCOMP_OK;
 }

@@ -128,6 +128,52 @@ def test_ssim_identity_at_full_frame_size(gpu):
     assert abs(gpu.ssim(d, gpu.decompress(out, n, shape), shape) - 1.0) < 1e-12
 
 
+# rows at every alignment of both volumes (odd widths alternate), the first and
+# last rows read by elements, 32- and 64-bit products (values on both sides of
+# 2^14, in the original only and in the decoded volume only), windows on both
+# sides of a wave's and a workgroup's
+@pytest.mark.parametrize("oa,od", [(0, 0), (1, 1), (0, 1), (1, 0)])
+@pytest.mark.parametrize("shape", [(7, 7, 7), (8, 21, 133), (13, 24, 136), (9, 11, 265)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_ssim_alignment_and_value_range(gpu, orc, shape, oa, od):
+    import torch
+    rng = np.random.default_rng(oa + 2 * od + sum(shape))
+    n = shape[0] * shape[1] * shape[2]
+    for big in (0, 1, 2):
+        a = rng.integers(0, 1 << 14, shape).astype(np.uint16)
+        b = _noisy(a, rng, 50)
+        b[b >= 1 << 14] = (1 << 14) - 1
+        if big:
+            (a if big == 1 else b)[tuple(rng.integers(0, k) for k in shape)] = 1 << 14
+        va, vb = (torch.zeros(n + 8, dtype=torch.int16, device="cuda")[o:o + n] for o in (oa, od))
+        va.copy_(_dev(a).view(-1))
+        vb.copy_(_dev(b).view(-1))
+        assert gpu.ssim(va, vb, shape) == pytest.approx(orc.ssim(a, b), rel=1e-10, abs=1e-13)
+
+
+# the grouped pass and its element-wise ends: dword-aligned at different heads,
+# volumes of different alignment, fewer elements than a group, sums of squares
+# on both sides of 32 bits, zeros in the original (no relative error there)
+@pytest.mark.parametrize("oa,od", [(0, 0), (1, 1), (0, 1), (3, 1)])
+@pytest.mark.parametrize("n", [1, 8, 9, 17, 4097, 8 * 512 * 1024 + 13])
+def test_metrics_alignment_and_value_range(gpu, n, oa, od):
+    import torch
+    rng = np.random.default_rng(n + oa)
+    for top in (3, 1 << 14, 65536):
+        a = rng.integers(0, top, n).astype(np.uint16)
+        d = rng.integers(0, top, n).astype(np.uint16)
+        va, vd = (torch.zeros(n + 8, dtype=torch.int16, device="cuda")[o:o + n] for o in (oa, od))
+        va.copy_(torch.from_numpy(a.view(np.int16)))
+        vd.copy_(torch.from_numpy(d.view(np.int16)))
+        s = gpu.error_stats(va, vd)
+        e = np.abs(d.astype(np.int64) - a)
+        assert (s["max_abs_err"], s["min_orig"], s["max_orig"]) == (e.max(), a.min(), a.max())
+        assert s["sum_sq_err"] == int((e * e).sum()) and s["sum_sq_dec"] == int((d.astype(np.int64) ** 2).sum())
+        nz = a != 0
+        want = (e[nz].astype(np.float32) / a[nz].astype(np.float32)).max() if nz.any() else np.float32(0)
+        assert s["max_rel_err"] == float(want)
+
+
 def test_ssim_rejects_volumes_without_a_window(gpu):
     import lscomp
     v = _dev(np.zeros((6, 10, 10), np.uint16))
