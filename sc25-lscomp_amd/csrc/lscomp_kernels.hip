@@ -21,11 +21,19 @@
 // coalesced loads (for dense streams one tile ahead), and each lane unpacks
 // its block and writes its rows.  Rate-0 blocks decode to zeros.  uint32 volumes run the same
 // kernels with the uint32 codec.
+#include <cstdlib>
 #include "lscomp_internal.h"
 
 namespace lsc {
 
 constexpr uint32_t kSpinLimit = 1u << 16;
+// Probes of a missing total before a workgroup forms it itself
+// (compress_small_tile); LSCOMP_HELP_PROBES in the environment sets another
+// number.
+static const uint32_t kHelpProbes = [] {
+    const char *e = std::getenv("LSCOMP_HELP_PROBES");
+    return e ? (uint32_t)std::strtoul(e, nullptr, 10) : 1024u;
+}();
 
 // 16 bytes at 4-byte alignment.  Volume rows and stream bytes are in general
 // only dword aligned (volumes and stream buffers at 4-byte alignment are
@@ -744,23 +752,45 @@ __device__ __forceinline__ void block_coords(const Item &it, uint32_t b, uint32_
     bz = rem - by * it.nbz;
 }
 
+// Called by one thread of each of n workgroups (or groups of workgroups): the
+// last one to arrive resets the counters and advances the epoch.
+__device__ __forceinline__ void count_done(Ctrl *ctrl, uint32_t epoch, uint32_t n)
+{
+    const uint32_t old = __hip_atomic_fetch_add(&ctrl->done_ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (old == n - 1) {
+        __hip_atomic_store(&ctrl->ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&ctrl->chunk.v, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (uint32_t c = 0; c < kMaxCounters; c++)
+            __hip_atomic_store(&ctrl->ctr[c].v, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&ctrl->done_ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&ctrl->epoch, (epoch + 1u) & kEpochMask, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
 __device__ __forceinline__ void finish_launch(Ctrl *ctrl, uint32_t epoch)
 {
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t old = __hip_atomic_fetch_add(&ctrl->done_ctr, 1u, __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT);
-        if (old == gridDim.x - 1) {
-            __hip_atomic_store(&ctrl->ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&ctrl->chunk.v, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-            for (uint32_t c = 0; c < kMaxCounters; c++)
-                __hip_atomic_store(&ctrl->ctr[c].v, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&ctrl->done_ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&ctrl->epoch, (epoch + 1u) & kEpochMask, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        }
+    if (threadIdx.x == 0) count_done(ctrl, epoch, gridDim.x);
+}
+
+// finish_launch for launches that hand out no tile ids.  More than 128
+// workgroups count on the kMaxCounters tile-id lines first, the last one of
+// each line on done_ctr: at the end of a small volume all of them arrive
+// together, and the atomics on one line take 13 ns each (256 tiles 11.2 -> 9.4
+// us); at 128 and fewer the second round trip costs as much as it saves (128
+// tiles 7.2 -> 7.7 us).
+__device__ __forceinline__ void finish_small(Ctrl *ctrl, uint32_t epoch)
+{
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    if (gridDim.x <= 128u) {
+        count_done(ctrl, epoch, gridDim.x);
+        return;
     }
+    const uint32_t c = blockIdx.x % kMaxCounters, n = (gridDim.x - c + kMaxCounters - 1u) / kMaxCounters;
+    if (__hip_atomic_fetch_add(&ctrl->ctr[c].v, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1)
+        count_done(ctrl, epoch, kMaxCounters);
 }
 
 // Dynamic tile ids (thread 0 of a workgroup only).  Tile k*nc + c is the k-th
@@ -1078,6 +1108,102 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void 
 {
     compress_tiles<CodecU16T<kTable, kKind>, TILE, kTable>(single, items, tile_items, total_tiles, d_total_tiles,
                                                                ctrl, status, sc);
+}
+
+// Compression of a single item of at most kSmallTiles tiles: one workgroup per
+// tile (tile = its index), without tickets, pipeline or prefix chain.  A
+// workgroup's block loads are its first instructions; it publishes its tile's
+// total, packs, and adds the totals of every tile before its own (at most 256
+// words, up to 4 per thread, read together), so the launch is three dependent
+// memory round trips (blocks, totals, stores).  Latency-bound: the pipelined
+// kernel spends a round trip on its start ticket, two empty iterations on
+// draining and a serialized ticket atomic per workgroup on the way (one 512 x
+// 512 frame lossless 10.2 -> 5.7 us, 16 of them 10.8 -> 7.4, one 2048 x 2048
+// frame lossy 11.6 -> 8.4).
+//
+// Forward progress does not depend on which workgroups are resident: one that
+// has found a tile's total missing for `help` probes forms that total itself
+// (the value its owner will publish too) and goes on, one missing tile at a
+// time, so every wait ends.
+template <int TILE, uint32_t W>
+struct SmallShared {
+    alignas(16) uint32_t pay[TILE * W + 8];
+    uint32_t hdr[TILE / 4];
+    uint32_t wsum[TILE / 64], lsum[TILE / 64];
+    uint32_t missing;
+};
+
+template <class C, int TILE>
+__device__ __forceinline__ void compress_small_tile(const Item &it, Ctrl *ctrl, uint64_t *status, uint32_t help)
+{
+    constexpr uint32_t kPer = kSmallTiles / TILE ? kSmallTiles / TILE : 1u;   // totals per thread at most
+    static_assert(kPer * TILE >= kSmallTiles, "every tile before the last one is read");
+    __shared__ SmallShared<TILE, C::kMaxWords> sh;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, t = blockIdx.x;
+    const uint32_t epoch_v = __hip_atomic_load(&ctrl->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // payload words of this thread's block of tile u (its header byte in hdr)
+    uint32_t D[C::kRegs], hdr = 0;
+    const auto block_words = [&](uint32_t u) -> uint32_t {
+        const uint32_t b = u * (uint32_t)TILE + tid;
+        hdr = 0;
+        if (b < it.nblocks) {
+            uint32_t bx, by, bz;
+            block_coords(it, b, bx, by, bz);
+            C::load(it, bx, by, bz, D);
+            hdr = C::header(D, it, ctrl);
+        }
+        return header_payload_bytes(hdr) >> 2;
+    };
+    const uint32_t words = block_words(t);
+    const uint32_t epoch = __builtin_amdgcn_readfirstlane(epoch_v);
+    ((uint8_t *)sh.hdr)[tid] = (uint8_t)hdr;
+    if (tid == 0) sh.missing = ~0u;
+    uint32_t agg;
+    const uint32_t off = tile_scan<TILE>(words, tid, sh.wsum, &agg);
+    if (tid == 0) st_relaxed(status + t, lb_word(epoch, LB_AGG, agg));
+    if (words) C::encode(D, hdr, it, &sh.pay[off]);
+
+    uint32_t sum = 0, open = 0;   // open: bit k is set while the total of tile tid + k * TILE is missing
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; k++) open |= tid + k * TILE < t ? 1u << k : 0u;
+    for (;;) {
+        for (uint32_t spins = 0; open != 0; spins++) {
+            uint64_t w[kPer];
+#pragma unroll
+            for (uint32_t k = 0; k < kPer; k++) w[k] = (open >> k) & 1u ? ld_relaxed(status + tid + k * TILE) : 0ull;
+#pragma unroll
+            for (uint32_t k = 0; k < kPer; k++)
+                if (((open >> k) & 1u) && (uint32_t)(w[k] >> 38) == epoch && ((uint32_t)(w[k] >> 36) & 3u) != LB_EMPTY) {
+                    sum += (uint32_t)w[k];
+                    open &= ~(1u << k);
+                }
+            if (open != 0 && spins >= help) break;
+            if (open != 0) __builtin_amdgcn_s_sleep(1);
+        }
+        if (open != 0) atomicMin(&sh.missing, tid + (uint32_t)__builtin_ctz(open) * TILE);
+        const uint32_t incl = wave_incl_scan(sum, lane);
+        if (lane == 63) sh.lsum[wave] = incl;
+        __syncthreads();
+        const uint32_t m = sh.missing;
+        if (m == ~0u) break;
+        __syncthreads();
+        if (tid == 0) sh.missing = ~0u;
+        uint32_t total;
+        (void)tile_scan<TILE>(block_words(m), tid, sh.wsum, &total);
+        if (tid == 0) st_relaxed(status + m, lb_word(epoch, LB_AGG, total));
+        __syncthreads();
+    }
+    uint32_t excl = 0;   // at most 256 tiles of 512 blocks of 32 words: 32 bits
+#pragma unroll
+    for (int v = 0; v < TILE / 64; v++) excl += sh.lsum[v];
+    store_tile<TILE>(it, t, agg, sh.hdr, sh.pay, excl, tid);
+    finish_small(ctrl, epoch);
+}
+
+template <class C, int TILE>
+__global__ __launch_bounds__(TILE) void compress_small_kernel(const Item it, Ctrl *ctrl, uint64_t *status, uint32_t help)
+{
+    compress_small_tile<C, TILE>(it, ctrl, status, help);
 }
 
 // ---------------------------------------------------------------------------
@@ -1760,6 +1886,52 @@ static bool use_pipe_decode(const Item &it)
     return dense_stream(it);
 }
 
+// Small compressions (compress_small_tile), any kind of settings.
+template <int TILE>
+static void launch_small_t(Item it, Ctrl *ctrl, uint64_t *status, hipStream_t stream)
+{
+    it.ntiles = (it.nblocks + TILE - 1) / TILE;
+    const dim3 grid(it.ntiles), block(TILE);
+    if (it.dec.flags & DEC_LOSSLESS)
+        hipLaunchKernelGGL((compress_small_kernel<CodecU16T<false, KIND_LOSSLESS>, TILE>), grid, block, 0, stream, it,
+                           ctrl, status, kHelpProbes);
+    else if (it.dec.flags & DEC_Q24)
+        hipLaunchKernelGGL((compress_small_kernel<CodecU16T<false, KIND_Q24>, TILE>), grid, block, 0, stream, it, ctrl,
+                           status, kHelpProbes);
+    else
+        hipLaunchKernelGGL((compress_small_kernel<CodecU16T<false>, TILE>), grid, block, 0, stream, it, ctrl, status,
+                           kHelpProbes);
+}
+
+template <int TILE>
+static void launch_small_u32_t(Item it, Ctrl *ctrl, uint64_t *status, hipStream_t stream)
+{
+    it.ntiles = (it.nblocks + TILE - 1) / TILE;
+    hipLaunchKernelGGL((compress_small_kernel<CodecU32, TILE>), dim3(it.ntiles), dim3(TILE), 0, stream, it, ctrl, status,
+                       kHelpProbes);
+}
+
+// Blocks per tile of a small compression: the smallest tile that keeps the
+// workgroups few, since a workgroup's own time grows with its waves (4096
+// blocks: 5.7 / 6.1 / 7.1 / 8.2 us at 64 / 128 / 256 / 512) and a launch's with
+// its workgroups (16384 blocks: 8.0 / 6.6 / 6.8 / 8.5; 44265 blocks at 256 /
+// 512: 6.4 / 7.1; 65536: 8.2 / 7.7).
+static uint32_t small_tile(uint32_t nblocks)
+{
+    return nblocks <= 64u * 64u ? 64u : nblocks <= 128u * 128u ? 128u : nblocks <= 256u * 192u ? 256u : 512u;
+}
+
+static hipError_t launch_small(const Item &it, Ctrl *ctrl, uint64_t *status, hipStream_t stream)
+{
+    switch (small_tile(it.nblocks)) {
+    case 64: launch_small_t<64>(it, ctrl, status, stream); break;
+    case 128: launch_small_t<128>(it, ctrl, status, stream); break;
+    case 256: launch_small_t<256>(it, ctrl, status, stream); break;
+    default: launch_small_t<512>(it, ctrl, status, stream); break;
+    }
+    return hipGetLastError();
+}
+
 template <int TILE>
 static hipError_t launch_t(bool compress, const Item &single, const Item *items, const uint32_t *tile_items, LaunchCfg cfg,
                            Ctrl *ctrl, uint64_t *status, hipStream_t stream)
@@ -2180,7 +2352,11 @@ hipError_t launch_u32(bool compress, const Item &it, LaunchCfg cfg, Ctrl *ctrl, 
     constexpr int T = (int)kTileU32, TD = (int)kTileU32Dec;
     if (cfg.tile != (uint32_t)(compress ? T : TD)) return hipErrorInvalidValue;
     const dim3 grid(cfg.grid);
-    if (compress) {
+    if (compress && it.ntiles <= kSmallTiles) {   // of 256 blocks
+        if (it.nblocks <= 64u * 64u) launch_small_u32_t<64>(it, ctrl, status, stream);
+        else if (it.nblocks <= 128u * 128u) launch_small_u32_t<128>(it, ctrl, status, stream);
+        else launch_small_u32_t<T>(it, ctrl, status, stream);
+    } else if (compress) {
         hipLaunchKernelGGL((compress_u32_kernel<T>), grid, dim3(T), 0, stream, it, ctrl, status, cfg.sched);
     } else if (it.ntiles <= kSmallTiles) {
         hipLaunchKernelGGL((decompress_u32_small_kernel<TD>), dim3(it.ntiles), dim3(TD), 0, stream, it, ctrl);
@@ -2200,7 +2376,10 @@ static hipError_t launch(bool compress, const Item &single, const Item *items, c
     switch (cfg.tile) {
     case 128: return launch_t<128>(compress, single, items, tile_items, cfg, ctrl, status, stream);
     case 256: return launch_t<256>(compress, single, items, tile_items, cfg, ctrl, status, stream);
-    case 512: return launch_t<512>(compress, single, items, tile_items, cfg, ctrl, status, stream);
+    case 512:
+        // one small volume at the default tile (another tile asks for that launch shape)
+        if (compress && !items && single.ntiles <= kSmallTiles) return launch_small(single, ctrl, status, stream);
+        return launch_t<512>(compress, single, items, tile_items, cfg, ctrl, status, stream);
     case kPipeTile:   // the pipelined decode of one dense volume with the offset phase only
         if (compress || items || !cfg.tile_off || cfg.off_mode != OFF_PHASE || !dense_stream(single))
             return hipErrorInvalidValue;
