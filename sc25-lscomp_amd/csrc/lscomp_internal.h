@@ -141,12 +141,14 @@ hipError_t launch_fill_u64(uint64_t *p, uint64_t n, uint64_t value, hipStream_t 
 // 4-wave ones on tiles of 256, and 6-11 % slower compressing); decompression
 // always computes tile offsets first (cfg.tile_off must be set).
 constexpr uint32_t kTileU32 = 256;
-// Decode geometry of a single uint16 volume.  At most kSmallTiles tiles: one
-// workgroup per tile that sums the header bytes before it.  A payload-dense
+// Small single volumes: at most kSmallTiles tiles compress, and at most
+// kSmallDecTiles tiles of 512 blocks decompress, with one workgroup per tile.
+// Decode geometry of a single uint16 volume above that: a payload-dense
 // stream (dense_stream) at the default and largest launch tile (512) with the
 // offset phase decodes in the pipelined decoder on tiles of kPipeTile blocks,
 // one 16-wave workgroup per CU.
 constexpr uint32_t kSmallTiles = 256;
+constexpr uint32_t kSmallDecTiles[2] = {704, 448};   // uint16, uint32
 constexpr uint32_t kPipeTile = 1024;
 constexpr uint32_t kTileU32Dec = 512;
 constexpr uint32_t tile_u32(bool compress) { return compress ? kTileU32 : kTileU32Dec; }

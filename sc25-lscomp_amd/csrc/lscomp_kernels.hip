@@ -1532,15 +1532,18 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void 
     finish_launch(ctrl, epoch);
 }
 
-// Decompression of a single item of at most kSmallTiles tiles: one workgroup
-// per tile, which sums the payload sizes of every block before its tile from
-// their header bytes itself (at most 255 * TILE bytes, 16-byte pieces strided
-// over the workgroup, four loads in flight per thread).  No workgroup waits
-// for another and no counter or epoch is used, so the launch is a chain of
-// three memory round trips (header bytes, payload, row stores) instead of the
-// offset phase's chunk ticket, header pass, look-back and tile ids ahead of
-// the decode.  The header bytes before a tile are read once per later tile,
-// but the whole header section is at most 128 KB and stays in L2.
+// Decompression of a small single item: one workgroup per tile, which sums the
+// payload sizes of every block before its tile from their header bytes itself
+// (16-byte pieces strided over the workgroup, four loads in flight per
+// thread).  No workgroup waits for another and no counter or epoch is used, so
+// the launch is a chain of three memory round trips (header bytes, payload,
+// row stores) instead of the offset phase's chunk ticket, header pass,
+// look-back and tile ids ahead of the decode.  The header bytes before a tile
+// are read once per later tile, from L2: the header section of 704 tiles of
+// 512 blocks is 352 KB.  That reading grows with the square of the volume (in
+// tiles of 512: 306 28.1 -> 12.3 us, 346 30.1 -> 15.2, 692 31.8 -> 26.4, 1024
+// 25.0 -> 35.7; uint32 306 32.5 -> 21.4, 346 31.6 -> 24.0, 605 33.0 -> 38.2),
+// hence the limits kSmallDecTiles.
 template <class C, int TILE>
 __device__ __forceinline__ void decompress_small_tiles(const Item &it, Ctrl *ctrl)
 {
@@ -1550,18 +1553,19 @@ __device__ __forceinline__ void decompress_small_tiles(const Item &it, Ctrl *ctr
     const uint32_t b = t * (uint32_t)TILE + tid;
     const bool valid = b < it.nblocks;
     const uint32_t hdr = valid ? (uint32_t)it.s_in[b] : 0u;
-    // payload words before this tile: at most 255 tiles of 512 blocks of 32
-    // words (or 256 blocks of 62), so 32 bits hold every partial sum
+    // payload words before this tile: at most 704 tiles of 512 blocks of
+    // at most 62 words, so 32 bits hold every partial sum
     uint32_t before = 0;
     const uint32_t npieces = t * ((uint32_t)TILE / 16u);
     for (uint32_t i = tid; i < npieces; i += 4u * TILE) {
-        uint32_t w[4];
+        uint4 x[4];   // whole pieces: every block before this tile exists
 #pragma unroll
         for (uint32_t k = 0; k < 4; k++) {
             const uint32_t j = i + k * (uint32_t)TILE;
-            w[k] = j < npieces ? words16(it, 16ull * j) : 0u;
+            x[k] = j < npieces ? ld16_a4(it.s_in + 16u * j) : make_uint4(0, 0, 0, 0);
         }
-        before += (w[0] + w[1]) + (w[2] + w[3]);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) before += (words4(x[k].x) + words4(x[k].y)) + (words4(x[k].z) + words4(x[k].w));
     }
     const uint32_t wtot = (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan(before, lane), 63);
     if (lane == 0) sh.wsum[1][wave] = wtot;
@@ -1596,6 +1600,13 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void 
     const Item it, Ctrl *ctrl)
 {
     decompress_small_tiles<CodecU16, TILE>(it, ctrl);
+}
+
+template <int TILE>
+__global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(2))) void decompress_u32_small_kernel(
+    const Item it, Ctrl *ctrl)
+{
+    decompress_small_tiles<CodecU32, TILE>(it, ctrl);
 }
 
 // Decompression of a single item with precomputed tile offsets, pipelined so
@@ -1921,6 +1932,28 @@ static uint32_t small_tile(uint32_t nblocks)
     return nblocks <= 64u * 64u ? 64u : nblocks <= 128u * 128u ? 128u : nblocks <= 256u * 192u ? 256u : 512u;
 }
 
+// The same for decompression, which has no counters to serialize on: 4096
+// blocks 4.5 / 4.9 / 5.4 / 5.7 us at 64 / 128 / 256 / 512, 16384 blocks 5.9 /
+// 5.3 / 5.3 / 6.1, 65536 blocks 12.7 / 10.4 / 7.3 / 7.7, 114075 blocks at 256 /
+// 512 12.6 / 10.9.
+template <int TILE>
+static void launch_small_decode_t(Item it, Ctrl *ctrl, hipStream_t stream)
+{
+    it.ntiles = (it.nblocks + TILE - 1) / TILE;
+    if (it.elem == 2)
+        hipLaunchKernelGGL((decompress_small_kernel<TILE>), dim3(it.ntiles), dim3(TILE), 0, stream, it, ctrl);
+    else
+        hipLaunchKernelGGL((decompress_u32_small_kernel<TILE>), dim3(it.ntiles), dim3(TILE), 0, stream, it, ctrl);
+}
+
+static void launch_small_decode(const Item &it, Ctrl *ctrl, hipStream_t stream)
+{
+    if (it.nblocks <= 4096u) launch_small_decode_t<64>(it, ctrl, stream);
+    else if (it.nblocks <= 16384u) launch_small_decode_t<128>(it, ctrl, stream);
+    else if (it.nblocks <= 65536u) launch_small_decode_t<256>(it, ctrl, stream);
+    else launch_small_decode_t<512>(it, ctrl, stream);
+}
+
 static hipError_t launch_small(const Item &it, Ctrl *ctrl, uint64_t *status, hipStream_t stream)
 {
     switch (small_tile(it.nblocks)) {
@@ -1958,6 +1991,8 @@ static hipError_t launch_t(bool compress, const Item &single, const Item *items,
         else if (items)
             hipLaunchKernelGGL((decompress_kernel<TILE, true>), grid, block, 0, stream, single, items, tile_items,
                                cfg.total_tiles, cfg.d_total_tiles, ctrl, status, (uint64_t *)nullptr, sc, 0u);
+        else if (TILE == 512 && single.ntiles <= kSmallDecTiles[0])
+            launch_small_decode(single, ctrl, stream);
         else if (single.ntiles <= kSmallTiles)
             hipLaunchKernelGGL((decompress_small_kernel<TILE>), dim3(single.ntiles), block, 0, stream, single, ctrl);
         else
@@ -2339,13 +2374,6 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(2))) void 
     decompress_pipe_tiles<CodecU32, TILE>(it, ctrl, status, tile_off, sc, phase);
 }
 
-template <int TILE>
-__global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(2))) void decompress_u32_small_kernel(
-    const Item it, Ctrl *ctrl)
-{
-    decompress_small_tiles<CodecU32, TILE>(it, ctrl);
-}
-
 hipError_t launch_u32(bool compress, const Item &it, LaunchCfg cfg, Ctrl *ctrl, uint64_t *status,
                       hipStream_t stream)
 {
@@ -2358,8 +2386,8 @@ hipError_t launch_u32(bool compress, const Item &it, LaunchCfg cfg, Ctrl *ctrl, 
         else launch_small_u32_t<T>(it, ctrl, status, stream);
     } else if (compress) {
         hipLaunchKernelGGL((compress_u32_kernel<T>), grid, dim3(T), 0, stream, it, ctrl, status, cfg.sched);
-    } else if (it.ntiles <= kSmallTiles) {
-        hipLaunchKernelGGL((decompress_u32_small_kernel<TD>), dim3(it.ntiles), dim3(TD), 0, stream, it, ctrl);
+    } else if (it.ntiles <= kSmallDecTiles[1]) {
+        launch_small_decode(it, ctrl, stream);
     } else {
         if (!cfg.tile_off) return hipErrorInvalidValue;
         const uint32_t phase = cfg.off_mode == OFF_PHASE ? 1u : 0u;

@@ -1,4 +1,4 @@
-"""Compression of small volumes (one workgroup per tile, no tile ids): byte-equal
+"""Small volumes (one workgroup per tile, no tile ids).  Compression: byte-equal
 to the oracle at the edges of the tile choice and of the path itself, over
 calls whose sizes go up and down on one scratch area, and with workgroups
 forming totals they find missing themselves (LSCOMP_HELP_PROBES=0: after the
@@ -45,6 +45,29 @@ def test_small_edges_u32(gpu, orc, n):
         assert st == 0
         out, got = gpu.compress_u32(torch.from_numpy(vol.view(np.int32)).cuda(), vol.shape, bins, p)
         assert got == refn and np.array_equal(out[:got].cpu().numpy(), ref)
+
+
+# decompression: the edges of its tile sizes (64, 128, 256, 512 blocks) and of
+# the path (704 tiles of 512 blocks; 448 for uint32), sparse and dense payloads
+@pytest.mark.parametrize("kind", ["sparse", "uniform"])
+@pytest.mark.parametrize("n", [1, 63, 65, 4096, 4097, 16384, 16385, 65536, 65537, 704 * 512, 704 * 512 + 1])
+def test_small_decode_edges(gpu, orc, kind, n):
+    import torch
+    vol = synth(kind, (1, 7, 8 * n - 3), seed=n)
+    for bins, p in (MODES["lossless"], MODES["b3-5-10-15_p0.5"]):
+        _, ref, refn = orc.compress(vol, bins, p)
+        _, want = orc.decompress(ref, vol.shape, bins)
+        got = gpu.decompress(torch.from_numpy(ref).cuda(), refn, vol.shape, bins)
+        assert np.array_equal(got.cpu().numpy().view(np.uint16), want)
+
+
+@pytest.mark.parametrize("n", [65, 4096, 4097, 16385, 65537, 448 * 512, 448 * 512 + 1])
+def test_small_decode_edges_u32(gpu, orc, n):
+    import torch
+    vol = np.random.default_rng(n).poisson(0.4, (1, 8, 8 * n - 2)).astype(np.uint32) << 12
+    _, ref, refn = orc.compress_u32(vol, (1, 1, 1, 1), 1.0)
+    got = gpu.decompress_u32(torch.from_numpy(ref).cuda(), refn, vol.shape)
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), vol)
 
 
 def test_small_missing_totals_are_formed(gpu):
