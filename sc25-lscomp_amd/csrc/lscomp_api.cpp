@@ -170,11 +170,12 @@ struct Scratch {
     uint64_t cap_tiles = 0;
     uint64_t *tile_off = nullptr;  // device, cap_tiles + 1 decode tile offsets
     uint64_t launches = 0;         // epochs used since the status words were cleared
-    Ctrl *host = nullptr;          // pinned readback of ctrl
+    CtrlHost *host = nullptr;      // pinned, written by the kernels
+    bool copy_head = false;        // a uint32 compression ran since the last wait_host
     void *aux = nullptr;           // device, kAuxKeep bytes (AuxLease), allocated at first use
     std::mutex mu;
 };
-static_assert(sizeof(Ctrl) >= 256 + kAuxHost, "the host readback area holds a Ctrl head and an AuxLease result");
+static_assert(sizeof(CtrlHost::aux) >= kAuxHost, "AuxLease results");
 
 std::mutex g_mu;
 std::map<std::pair<int, hipStream_t>, Scratch *> g_scratch;
@@ -191,12 +192,14 @@ Scratch *get_scratch(hipStream_t stream)
     s->device = dev;
     s->stream = stream;
     if (hipMalloc((void **)&s->ctrl, sizeof(Ctrl)) != hipSuccess ||
-        hipHostMalloc((void **)&s->host, sizeof(Ctrl), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void **)&s->host, sizeof(CtrlHost), hipHostMallocDefault) != hipSuccess) {
         if (s->ctrl) (void)hipFree(s->ctrl);
         delete s;
         return nullptr;
     }
-    if (launch_fill_u64((uint64_t *)s->ctrl, sizeof(Ctrl) / 8, 0, stream) != hipSuccess) {
+    std::memset((void *)s->host, 0, sizeof(CtrlHost));
+    if (launch_fill_u64((uint64_t *)s->ctrl, sizeof(Ctrl) / 8, 0, stream) != hipSuccess ||
+        launch_fill_u64((uint64_t *)&s->ctrl->flags, 1, (uint64_t)(uintptr_t)s->host->flags, stream) != hipSuccess) {
         (void)hipFree(s->ctrl);
         (void)hipHostFree(s->host);
         delete s;
@@ -244,23 +247,31 @@ int count_launch(Scratch *s)
     return LSCOMP_OK;
 }
 
-int read_ctrl(Scratch *s)
+// Waits for the stream; s->host then holds what its launches left.
+int wait_host(Scratch *s)
 {
-    int st = hip_fail(hipMemcpyAsync(s->host, s->ctrl, kCtrlHead, hipMemcpyDeviceToHost, s->stream),
-                      "hipMemcpyAsync");
-    if (st) return st;
+    if (s->copy_head) {
+        const int st = hip_fail(hipMemcpyAsync(s->host, s->ctrl, kCtrlHead, hipMemcpyDeviceToHost, s->stream),
+                                "hipMemcpyAsync");
+        if (st) return st;
+        s->copy_head = false;
+    }
     return hip_fail(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
 }
 
-// Returns the status for sticky error bits and clears them.
+// Returns the status for sticky error bits and clears them (after wait_host).
 int take_errors(Scratch *s)
 {
-    const uint32_t e = s->host->error;
+    volatile uint32_t *f = s->host->flags;
+    const uint32_t e = s->host->error | (f[0] ? 1u : 0u) | (f[1] ? 2u : 0u);
+    static_assert(ERRF_CORRUPT == 1u && ERRF_TIMEOUT == 2u && ERRF_RANGE == 4u, "flag words by bit");
     if (!e) return LSCOMP_OK;
     int st = hip_fail(launch_fill_u64((uint64_t *)&s->ctrl->error, 1, 0, s->stream), "fill");
     if (st) return st;
     st = hip_fail(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
     if (st) return st;
+    f[0] = f[1] = f[2] = 0;
+    s->host->error = 0;
     if (e & ERRF_TIMEOUT) return LSCOMP_ERR_INTERNAL;
     if (e & ERRF_RANGE) return LSCOMP_ERR_RANGE;
     return LSCOMP_ERR_CORRUPT;
@@ -278,7 +289,7 @@ AuxLease::AuxLease(hipStream_t stream, size_t bytes, size_t host_bytes) : stream
         return;
     }
     lk_ = std::unique_lock<std::mutex>(s->mu);
-    host_ = (uint8_t *)s->host + 256;   // beside the control head's readback
+    host_ = s->host->aux;
     if (bytes > kAuxKeep) {
         st_ = hip_fail(hipMalloc(&dev_, bytes), "hipMalloc");
         own_ = st_ == LSCOMP_OK;
@@ -387,6 +398,7 @@ int launch_item_u32(Scratch *s, Item &it, bool compress)
     cfg.sched.win = default_window(cfg.tile);
     if (compress) {
         if (!it.result) it.result = &s->ctrl->result;
+        s->copy_head = true;
     } else {
         cfg.tile_off = s->tile_off;
         cfg.off_mode = g_decode_mode.load() == 2 ? OFF_KERNEL : OFF_PHASE;
@@ -409,7 +421,7 @@ int launch_item(Scratch *s, Item &it, bool compress, const Shape &shape)
     if (st) return st;
     const LaunchCfg cfg = make_cfg(it.ntiles, compress, false, shape);
     if (compress) {
-        if (!it.result) it.result = &s->ctrl->result;
+        if (!it.result) it.result = &s->host->size;
         return hip_fail(launch_compress(it, nullptr, nullptr, cfg, s->ctrl, s->status, s->stream), "compress launch");
     }
     LaunchCfg dcfg = cfg;
@@ -476,9 +488,9 @@ int lscomp_compress_u16(const uint16_t *d_in, uint8_t *d_out, size_t out_capacit
     std::lock_guard<std::mutex> lk(s->mu);
     st = launch_item(s, it, true, shape);
     if (st) return st;
-    st = read_ctrl(s);
+    st = wait_host(s);
     if (st) return st;
-    *out_bytes = (size_t)s->host->result;
+    *out_bytes = (size_t)*(volatile uint64_t *)&s->host->size;
     st = take_errors(s);
     if (st) return st;
     return *out_bytes > out_capacity ? LSCOMP_ERR_CAPACITY : LSCOMP_OK;
@@ -509,7 +521,7 @@ int lscomp_decompress_u16(uint16_t *d_out, const uint8_t *d_in, size_t in_bytes,
     std::lock_guard<std::mutex> lk(s->mu);
     st = launch_item(s, it, false, shape);
     if (st) return st;
-    st = read_ctrl(s);
+    st = wait_host(s);
     if (st) return st;
     return take_errors(s);
 }
@@ -547,9 +559,9 @@ int lscomp_compress_u32(const uint32_t *d_in, uint8_t *d_out, size_t out_capacit
     std::lock_guard<std::mutex> lk(s->mu);
     st = launch_item_u32(s, it, true);
     if (st) return st;
-    st = read_ctrl(s);
+    st = wait_host(s);
     if (st) return st;
-    *out_bytes = (size_t)s->host->result;
+    *out_bytes = (size_t)*(volatile uint64_t *)&s->host->result;
     st = take_errors(s);
     if (st) return st;
     return *out_bytes > out_capacity ? LSCOMP_ERR_CAPACITY : LSCOMP_OK;
@@ -578,7 +590,7 @@ int lscomp_decompress_u32(uint32_t *d_out, const uint8_t *d_in, size_t in_bytes,
     std::lock_guard<std::mutex> lk(s->mu);
     st = launch_item_u32(s, it, false);
     if (st) return st;
-    st = read_ctrl(s);
+    st = wait_host(s);
     if (st) return st;
     return take_errors(s);
 }
@@ -588,7 +600,7 @@ int lscomp_stream_status(hipStream_t stream)
     Scratch *s = get_scratch(stream);
     if (!s) return LSCOMP_ERR_HIP;
     std::lock_guard<std::mutex> lk(s->mu);
-    int st = read_ctrl(s);
+    int st = wait_host(s);
     if (st) return st;
     return take_errors(s);
 }

@@ -363,7 +363,7 @@ int lscomp_plan_status(lscomp_plan p, hipStream_t stream)
 {
     if (!p) return LSCOMP_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lk(p->mu);
-    int st = hip_fail(hipMemcpyAsync(p->h_ctrl, p->ctrl, kCtrlHead, hipMemcpyDeviceToHost, stream), "readback");
+    int st = hip_fail(hipMemcpyAsync(&p->h_ctrl->error, &p->ctrl->error, sizeof(uint32_t), hipMemcpyDeviceToHost, stream), "readback");
     if (st) return st;
     st = hip_fail(hipStreamSynchronize(stream), "hipStreamSynchronize");
     if (st) return st;

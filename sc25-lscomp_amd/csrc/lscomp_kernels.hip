@@ -70,6 +70,17 @@ __device__ __forceinline__ void st_relaxed(uint64_t *p, uint64_t v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Flags the launch (one ERRF_* bit), also where the host reads without a copy.
+// Not for the hot loops of compression, which set Ctrl::error alone (this code
+// in the look-back took uint32 compression 740 -> 745 us): finish_launch
+// passes a time-out on, and the host copies the word for ERRF_RANGE.
+__device__ __forceinline__ void flag_error(Ctrl *ctrl, uint32_t bit)
+{
+    __hip_atomic_fetch_or(&ctrl->error, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t *h = ctrl->flags;
+    if (h) __hip_atomic_store(h + __builtin_ctz(bit), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Inclusive scan over the wave's 64 lanes with DPP moves: shifts by 1, 2, 4 and
 // 8 lanes within each row of 16, then row 0's (row 2's) last lane added to row
 // 1 (row 3) and lane 31 added to rows 2 and 3.  Lanes a move does not reach
@@ -771,7 +782,12 @@ __device__ __forceinline__ void count_done(Ctrl *ctrl, uint32_t epoch, uint32_t 
 __device__ __forceinline__ void finish_launch(Ctrl *ctrl, uint32_t epoch)
 {
     __syncthreads();
-    if (threadIdx.x == 0) count_done(ctrl, epoch, gridDim.x);
+    if (threadIdx.x == 0) {
+        // a time-out of a look-back is flagged by this thread, so it is seen here
+        if (__hip_atomic_load(&ctrl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERRF_TIMEOUT)
+            flag_error(ctrl, ERRF_TIMEOUT);
+        count_done(ctrl, epoch, gridDim.x);
+    }
 }
 
 // finish_launch for launches that hand out no tile ids.  More than 128
@@ -1281,7 +1297,7 @@ __device__ __forceinline__ uint64_t off_value(const uint64_t *tile_off, uint32_t
         if (spins > kSpinLimit ||
             ((spins & 63u) == 0 &&
              (__hip_atomic_load(&ctrl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERRF_TIMEOUT))) {
-            __hip_atomic_fetch_or(&ctrl->error, ERRF_TIMEOUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            flag_error(ctrl, ERRF_TIMEOUT);
             v = ~0ull >> 3;
             break;
         }
@@ -1516,8 +1532,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void 
             __builtin_amdgcn_s_setprio(2);
             store_block<false>(it, bx, by, bz, D);
             __builtin_amdgcn_s_setprio(0);
-            if (bad) __hip_atomic_fetch_or(&ctrl->error, ERRF_CORRUPT, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
+            if (bad) flag_error(ctrl, ERRF_CORRUPT);
         }
         __syncthreads();
         if (tid == 0) {
@@ -1591,7 +1606,7 @@ __device__ __forceinline__ void decompress_small_tiles(const Item &it, Ctrl *ctr
         uint32_t bx, by, bz;
         block_coords(it, b, bx, by, bz);
         C::store(it, bx, by, bz, D);
-        if (bad) __hip_atomic_fetch_or(&ctrl->error, ERRF_CORRUPT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (bad) flag_error(ctrl, ERRF_CORRUPT);
     }
 }
 
@@ -1747,7 +1762,7 @@ __device__ __forceinline__ void decompress_pipe_tiles(const Item it_arg, Ctrl *c
             uint32_t bx, by, bz;
             block_coords(it, b, bx, by, bz);
             C::store(it, bx, by, bz, D);
-            if (bad) __hip_atomic_fetch_or(&ctrl->error, ERRF_CORRUPT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (bad) flag_error(ctrl, ERRF_CORRUPT);
         }
         __syncthreads();   // t's payload has left LDS; t1's is visible
         if (t1_start == ~0u) {   // 5. t1 did not fit beside t (or is large): stage it now
@@ -2198,7 +2213,7 @@ __device__ __forceinline__ void serve_consume(const SrvArgs &a, Ctrl *ctrl, uint
                 if ((c & 1u) && (uint64_t)n >= (c >> 1)) st = 2;
                 // closed above n, yet n's word never shows: give up (bounded wait)
                 if ((c & 1u) && st == 0 && ++late > kSpinLimit) {
-                    __hip_atomic_fetch_or(&ctrl->error, ERRF_TIMEOUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    flag_error(ctrl, ERRF_TIMEOUT);
                     st = 2;
                 }
             }
