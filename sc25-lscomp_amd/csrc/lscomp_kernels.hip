@@ -113,6 +113,13 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v)
 // ---------------------------------------------------------------------------
 // Block gather / scatter with zero padding (cuLSZ_kernel.cu:877-896, 1629-1640).
 // ---------------------------------------------------------------------------
+// kRows: the general code, or the code for volumes of align ALIGN2 alone with
+// their common case first.  Single volumes have a kernel of their own for it:
+// that case in the general kernel, and a kernel for dword rows alone, both took
+// the even widths longer (600 x 1813 x 1558 lossy compression 692 -> 714 us,
+// 512 uneven frames 321 -> 330).
+enum : int { ROWS_ANY = 0, ROWS_ODD = 1 };
+template <int kRows>
 __device__ __forceinline__ void load_block(const Item &it, uint32_t bx, uint32_t by, uint32_t bz,
                                            uint32_t D[32])
 {
@@ -120,7 +127,7 @@ __device__ __forceinline__ void load_block(const Item &it, uint32_t bx, uint32_t
     const uint16_t *p = it.vol_in + ((uint64_t)bx * it.y + y0) * it.z + z0;
     const uint32_t ny = it.y - y0 < 8u ? it.y - y0 : 8u;   // rows inside the volume
     const uint32_t nz = it.z - z0 < 8u ? it.z - z0 : 8u;   // columns inside the volume
-    if (it.align != ALIGN2) {
+    if (kRows == ROWS_ANY && it.align != ALIGN2) {
         // 16-byte row loads; global_load_dwordx4 needs only dword alignment, so
         // rows of 4-byte-aligned volumes (z even) load whole.  A block at the
         // end of a row (nz < 8, even) loads 16 bytes as well while they lie
@@ -179,6 +186,55 @@ __device__ __forceinline__ void load_block(const Item &it, uint32_t bx, uint32_t
         // elements past z; rows whose bytes would leave the volume (its first
         // and last rows) load by elements.
         const uint16_t *vol_end = it.vol_in + (uint64_t)it.x * it.y * it.z;
+        // The common case, z odd and a wave of whole-height blocks inside the
+        // volume whose rows have the same parities (they differ only between
+        // frames): one 16-byte load a row, from the dword boundary at or before
+        // its first element.  A row at 2 mod 4 then lacks its last element,
+        // which is the low half of the next lane's first word (v_mov_b32 with
+        // wave_shl:1): the next lane holds the next block of the row, since the
+        // block at a row's end has at most 7 elements here; only lane 63 loads
+        // it.  600 x 1813 x 1557 lossless 1.03 -> 0.77 ms and lossy 1.01 -> 0.74
+        // against the code below, which loads the 20 bytes of such a row by two
+        // instructions and tests every row.
+        const bool inside = ny == 8u && p > it.vol_in && p + 7ull * it.z + 9 <= vol_end;
+        const uint32_t u = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p >> 1) & 1u;
+        if (kRows == ROWS_ODD && (it.z & 1u) && __ballot(!inside || (((uint32_t)(uintptr_t)p >> 1) & 1u) != u) == 0) {
+            uint4 t[8];
+            uint32_t e[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int r = 0; r < 8; r++) t[r] = ld16_a4(p + (uint64_t)r * it.z - ((u ^ (uint32_t)r) & 1u));
+            if ((threadIdx.x & 63u) == 63u) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) e[k] = p[(uint64_t)(2 * k + (u ^ 1u)) * it.z + 7];
+            }
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+                uint32_t d0 = t[r].x, d1 = t[r].y, d2 = t[r].z, d3 = t[r].w;
+                if ((u ^ (uint32_t)r) & 1u) {   // uniform
+                    const uint32_t next = (uint32_t)__builtin_amdgcn_update_dpp((int)e[r >> 1], (int)d0, 0x130, 0xf, 0xf, false);
+                    d0 = __builtin_amdgcn_alignbit(d1, d0, 16);
+                    d1 = __builtin_amdgcn_alignbit(d2, d1, 16);
+                    d2 = __builtin_amdgcn_alignbit(d3, d2, 16);
+                    d3 = __builtin_amdgcn_alignbit(next, d3, 16);
+                }
+                D[4 * r] = d0;
+                D[4 * r + 1] = d1;
+                D[4 * r + 2] = d2;
+                D[4 * r + 3] = d3;
+            }
+            if (nz != 8u) {   // a block at a row end: clear the elements past z
+                const uint32_t m0 = nz > 1u ? ~0u : 0xffffu, m1 = nz > 3u ? ~0u : nz > 2u ? 0xffffu : 0u,
+                               m2 = nz > 5u ? ~0u : nz > 4u ? 0xffffu : 0u, m3 = nz > 6u ? 0xffffu : 0u;
+#pragma unroll
+                for (int r = 0; r < 8; r++) {
+                    D[4 * r] &= m0;
+                    D[4 * r + 1] &= m1;
+                    D[4 * r + 2] &= m2;
+                    D[4 * r + 3] &= m3;
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int r = 0; r < 8; r++) {
             const bool rv = (uint32_t)r < ny;
@@ -223,7 +279,8 @@ __device__ __forceinline__ void load_block(const Item &it, uint32_t bx, uint32_t
 // boundary as one 16-byte store: CSSI-shaped lossless decode (pipelined
 // decoder) 0.791 -> 0.765 ms.  The sparse decoder, whose row stores run at
 // raised wave priority, keeps the 12 + 4-byte form (0.707 against 0.719 ms).
-template <bool kSplit16>
+// kRows: as for load_block.
+template <bool kSplit16, int kRows = ROWS_ANY>
 __device__ __forceinline__ void store_block(const Item &it, uint32_t bx, uint32_t by, uint32_t bz,
                                             const uint32_t D[32])
 {
@@ -231,7 +288,7 @@ __device__ __forceinline__ void store_block(const Item &it, uint32_t bx, uint32_
     uint16_t *p = it.vol_out + ((uint64_t)bx * it.y + y0) * it.z + z0;
     const uint32_t ny = it.y - y0 < 8u ? it.y - y0 : 8u;
     const uint32_t nz = it.z - z0 < 8u ? it.z - z0 : 8u;
-    if (it.align != ALIGN2) {
+    if (kRows == ROWS_ANY && it.align != ALIGN2) {
         // z is even here, so nz is 2, 4, 6 or 8.  A row of 6 or 8 elements
         // stores its first 12 bytes, one of 2 or 4 its first dword; rows of 8
         // and of 4 then store their last dword with one shared instruction.
@@ -290,6 +347,50 @@ __device__ __forceinline__ void store_block(const Item &it, uint32_t bx, uint32_
             if (tail) q32[tail_at] = nz == 8u ? d3 : d1;
         }
     } else {
+        // The common case (load_block): a row at 2 mod 4 stores 16 bytes from its
+        // second element on, the last of them the next lane's first element.
+        // The first lane of a wave or of a row stores its own first element,
+        // lane 63 its elements 1 .. 7, the block at a row's end (nz is odd
+        // here) its pairs.  Pipelined decoder, 600 x 1813 x 1557 lossless 796
+        // -> 697 us; in the sparse one 718 -> 727, which keeps the five stores.
+        // (The same for dword rows, every lane storing the 16 bytes at its
+        // next 16-byte boundary, took 600 x 1813 x 1558 from 689 to 741 us.)
+        const uint32_t par = ((uint32_t)(uintptr_t)p >> 1) & 1u, u = __builtin_amdgcn_readfirstlane(par);
+        if (kRows == ROWS_ODD && (it.z & 1u) && __ballot(ny != 8u || par != u) == 0) {
+            const uint32_t lane = threadIdx.x & 63u;
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+                uint16_t *q = p + (uint64_t)r * it.z;
+                uint32_t d[4] = {D[4 * r], D[4 * r + 1], D[4 * r + 2], D[4 * r + 3]};
+                if (((u ^ (uint32_t)r) & 1u) == 0) {   // uniform
+                    if (nz == 8u) {
+                        st16_a4(q, make_uint4(d[0], d[1], d[2], d[3]));
+                    } else {
+                        uint32_t *m = (uint32_t *)q;
+                        if (nz > 1u) m[0] = d[0];
+                        if (nz > 3u) m[1] = d[1];
+                        if (nz > 5u) m[2] = d[2];
+                        q[nz - 1] = (uint16_t)(nz == 1u ? d[0] : nz == 3u ? d[1] : nz == 5u ? d[2] : d[3]);
+                    }
+                } else {
+                    const uint32_t next = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)d[0], 0x130, 0xf, 0xf, false);
+                    const uint32_t first = d[0];
+#pragma unroll
+                    for (int c = 0; c < 3; c++) d[c] = __builtin_amdgcn_alignbit(d[c + 1], d[c], 16);
+                    uint32_t *m = (uint32_t *)(q + 1);   // dword boundary
+                    if (nz == 8u && lane != 63u) {
+                        st16_a4(m, make_uint4(d[0], d[1], d[2], __builtin_amdgcn_alignbit(next, d[3], 16)));
+                    } else {
+                        if (nz > 2u) m[0] = d[0];
+                        if (nz > 4u) m[1] = d[1];
+                        if (nz > 6u) m[2] = d[2];
+                        if (nz == 8u) q[7] = (uint16_t)(d[3] >> 16);
+                    }
+                    if (lane == 0u || bz == 0u) q[0] = (uint16_t)first;
+                }
+            }
+            return;
+        }
         // Rows only 2-byte aligned: a row at a 4-byte boundary stores 16 bytes, a
         // row at 2 mod 4 its first element, the next pairs as dwords and its last
         // element; a block at a row end stores its nz elements the same way
@@ -420,13 +521,13 @@ __device__ __forceinline__ void store_block_u32(const Item &it, uint32_t bx, uin
 // store.  kMem: the item descriptors live in device memory (table mode), so
 // per-block parameters are read with indexed loads (sel4).  kKind: KIND_* of
 // every item (block_header).
-template <bool kMem, int kKind = KIND_ANY>
+template <bool kMem, int kKind = KIND_ANY, int kRows = ROWS_ANY>
 struct CodecU16T {
     static constexpr int kRegs = 32;              // 64 values as packed pairs
     static constexpr uint32_t kMaxWords = 32;     // 16 planes x 8 bytes
     __device__ __forceinline__ static void load(const Item &it, uint32_t bx, uint32_t by, uint32_t bz, uint32_t R[kRegs])
     {
-        load_block(it, bx, by, bz, R);
+        load_block<kRows>(it, bx, by, bz, R);
     }
     __device__ __forceinline__ static uint32_t header(const uint32_t R[kRegs], const Item &it, Ctrl *)
     {
@@ -443,7 +544,7 @@ struct CodecU16T {
     }
     __device__ __forceinline__ static void store(const Item &it, uint32_t bx, uint32_t by, uint32_t bz, const uint32_t R[kRegs])
     {
-        store_block<true>(it, bx, by, bz, R);
+        store_block<true, kRows>(it, bx, by, bz, R);
     }
 };
 
@@ -1117,12 +1218,12 @@ __device__ __forceinline__ void compress_tiles(const Item single, const Item *__
 // kKind: KIND_* of every item.  The general kernel's code for every kind of
 // settings costs scalar register spills: lossless CSSI compression was 2-3 %
 // slower in it than in its own kernel.
-template <int TILE, bool kTable, int kKind = KIND_ANY>
+template <int TILE, bool kTable, int kKind = KIND_ANY, int kRows = ROWS_ANY>
 __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void compress_kernel(
     const Item single, const Item *__restrict__ items, const uint32_t *__restrict__ tile_items, uint32_t total_tiles,
     const uint32_t *d_total_tiles, Ctrl *ctrl, uint64_t *status, Sched sc)
 {
-    compress_tiles<CodecU16T<kTable, kKind>, TILE, kTable>(single, items, tile_items, total_tiles, d_total_tiles,
+    compress_tiles<CodecU16T<kTable, kKind, kRows>, TILE, kTable>(single, items, tile_items, total_tiles, d_total_tiles,
                                                                ctrl, status, sc);
 }
 
@@ -1783,11 +1884,11 @@ __device__ __forceinline__ void decompress_pipe_tiles(const Item it_arg, Ctrl *c
     finish_launch(ctrl, epoch);
 }
 
-template <int TILE>
+template <int TILE, int kRows = ROWS_ANY>
 __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void decompress_pipe_kernel(
     const Item it, Ctrl *ctrl, uint64_t *status, uint64_t *__restrict__ tile_off, Sched sc, uint32_t phase)
 {
-    decompress_pipe_tiles<CodecU16, TILE>(it, ctrl, status, tile_off, sc, phase);
+    decompress_pipe_tiles<CodecU16T<false, KIND_ANY, kRows>, TILE>(it, ctrl, status, tile_off, sc, phase);
 }
 
 // ---------------------------------------------------------------------------
@@ -1980,6 +2081,24 @@ static hipError_t launch_small(const Item &it, Ctrl *ctrl, uint64_t *status, hip
     return hipGetLastError();
 }
 
+// One volume on the pipelined kernel of its kind of settings and alignment.
+template <int TILE, int kRows>
+static void launch_compress_t(const Item &it, const LaunchCfg &cfg, Ctrl *ctrl, uint64_t *status, hipStream_t stream)
+{
+    const dim3 grid(cfg.grid), block(TILE);
+    const Item *const none = nullptr;
+    const uint32_t *const no_map = nullptr;
+    if (it.dec.flags & DEC_LOSSLESS)
+        hipLaunchKernelGGL((compress_kernel<TILE, false, KIND_LOSSLESS, kRows>), grid, block, 0, stream, it, none, no_map,
+                           cfg.total_tiles, cfg.d_total_tiles, ctrl, status, cfg.sched);
+    else if (it.dec.flags & DEC_Q24)
+        hipLaunchKernelGGL((compress_kernel<TILE, false, KIND_Q24, kRows>), grid, block, 0, stream, it, none, no_map,
+                           cfg.total_tiles, cfg.d_total_tiles, ctrl, status, cfg.sched);
+    else
+        hipLaunchKernelGGL((compress_kernel<TILE, false, KIND_ANY, kRows>), grid, block, 0, stream, it, none, no_map,
+                           cfg.total_tiles, cfg.d_total_tiles, ctrl, status, cfg.sched);
+}
+
 template <int TILE>
 static hipError_t launch_t(bool compress, const Item &single, const Item *items, const uint32_t *tile_items, LaunchCfg cfg,
                            Ctrl *ctrl, uint64_t *status, hipStream_t stream)
@@ -1990,15 +2109,10 @@ static hipError_t launch_t(bool compress, const Item &single, const Item *items,
         if (items)
             hipLaunchKernelGGL((compress_kernel<TILE, true>), grid, block, 0, stream, single, items, tile_items,
                                cfg.total_tiles, cfg.d_total_tiles, ctrl, status, sc);
-        else if (single.dec.flags & DEC_LOSSLESS)
-            hipLaunchKernelGGL((compress_kernel<TILE, false, KIND_LOSSLESS>), grid, block, 0, stream, single, items,
-                               tile_items, cfg.total_tiles, cfg.d_total_tiles, ctrl, status, sc);
-        else if (single.dec.flags & DEC_Q24)
-            hipLaunchKernelGGL((compress_kernel<TILE, false, KIND_Q24>), grid, block, 0, stream, single, items,
-                               tile_items, cfg.total_tiles, cfg.d_total_tiles, ctrl, status, sc);
+        else if (single.align == ALIGN2)
+            launch_compress_t<TILE, ROWS_ODD>(single, cfg, ctrl, status, stream);
         else
-            hipLaunchKernelGGL((compress_kernel<TILE, false>), grid, block, 0, stream, single, items, tile_items,
-                               cfg.total_tiles, cfg.d_total_tiles, ctrl, status, sc);
+            launch_compress_t<TILE, ROWS_ANY>(single, cfg, ctrl, status, stream);
     } else {
         if (items && cfg.tile_off)
             hipLaunchKernelGGL((decompress_kernel<TILE, true, true>), grid, block, 0, stream, single, items,
@@ -2014,7 +2128,10 @@ static hipError_t launch_t(bool compress, const Item &single, const Item *items,
         {
             const uint32_t phase = cfg.tile_off && cfg.off_mode == OFF_PHASE ? 1u : 0u;
             if (cfg.tile_off && !phase) launch_offsets<TILE>(single, cfg, ctrl, status, stream);
-            if (cfg.tile_off && use_pipe_decode(single))
+            if (cfg.tile_off && use_pipe_decode(single) && single.align == ALIGN2)
+                hipLaunchKernelGGL((decompress_pipe_kernel<TILE, ROWS_ODD>), grid, block, 0, stream, single, ctrl, status,
+                                   cfg.tile_off, sc, phase);
+            else if (cfg.tile_off && use_pipe_decode(single))
                 hipLaunchKernelGGL((decompress_pipe_kernel<TILE>), grid, block, 0, stream, single, ctrl, status,
                                    cfg.tile_off, sc, phase);
             else if (cfg.tile_off)
@@ -2426,8 +2543,12 @@ static hipError_t launch(bool compress, const Item &single, const Item *items, c
     case kPipeTile:   // the pipelined decode of one dense volume with the offset phase only
         if (compress || items || !cfg.tile_off || cfg.off_mode != OFF_PHASE || !dense_stream(single))
             return hipErrorInvalidValue;
-        hipLaunchKernelGGL((decompress_pipe_kernel<kPipeTile>), dim3(cfg.grid), dim3(kPipeTile), 0, stream, single,
-                           ctrl, status, cfg.tile_off, cfg.sched, 1u);
+        if (single.align == ALIGN2)
+            hipLaunchKernelGGL((decompress_pipe_kernel<kPipeTile, ROWS_ODD>), dim3(cfg.grid), dim3(kPipeTile), 0, stream,
+                               single, ctrl, status, cfg.tile_off, cfg.sched, 1u);
+        else
+            hipLaunchKernelGGL((decompress_pipe_kernel<kPipeTile>), dim3(cfg.grid), dim3(kPipeTile), 0, stream, single,
+                               ctrl, status, cfg.tile_off, cfg.sched, 1u);
         return hipGetLastError();
     default: return hipErrorInvalidValue;
     }
