@@ -186,8 +186,8 @@ __device__ __forceinline__ void load_block(const Item &it, uint32_t bx, uint32_t
         // elements past z; rows whose bytes would leave the volume (its first
         // and last rows) load by elements.
         const uint16_t *vol_end = it.vol_in + (uint64_t)it.x * it.y * it.z;
-        // The common case, z odd and a wave of whole-height blocks inside the
-        // volume whose rows have the same parities (they differ only between
+        // The common case, z odd and a wave of blocks inside the volume (not
+        // in its first or last row) whose rows have the same parities (they differ only between
         // frames): one 16-byte load a row, from the dword boundary at or before
         // its first element.  A row at 2 mod 4 then lacks its last element,
         // which is the low half of the next lane's first word (v_mov_b32 with
@@ -196,16 +196,27 @@ __device__ __forceinline__ void load_block(const Item &it, uint32_t bx, uint32_t
         // it.  600 x 1813 x 1557 lossless 1.03 -> 0.77 ms and lossy 1.01 -> 0.74
         // against the code below, which loads the 20 bytes of such a row by two
         // instructions and tests every row.
-        const bool inside = ny == 8u && p > it.vol_in && p + 7ull * it.z + 9 <= vol_end;
+        const bool inside = p > it.vol_in && p + (uint64_t)(ny - 1u) * it.z + 9 <= vol_end;
         const uint32_t u = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p >> 1) & 1u;
         if (kRows == ROWS_ODD && (it.z & 1u) && __ballot(!inside || (((uint32_t)(uintptr_t)p >> 1) & 1u) != u) == 0) {
             uint4 t[8];
             uint32_t e[4] = {0, 0, 0, 0};
+            if (__ballot(ny != 8u) == 0) {
 #pragma unroll
-            for (int r = 0; r < 8; r++) t[r] = ld16_a4(p + (uint64_t)r * it.z - ((u ^ (uint32_t)r) & 1u));
-            if ((threadIdx.x & 63u) == 63u) {
+                for (int r = 0; r < 8; r++) t[r] = ld16_a4(p + (uint64_t)r * it.z - ((u ^ (uint32_t)r) & 1u));
+                if ((threadIdx.x & 63u) == 63u) {
 #pragma unroll
-                for (int k = 0; k < 4; k++) e[k] = p[(uint64_t)(2 * k + (u ^ 1u)) * it.z + 7];
+                    for (int k = 0; k < 4; k++) e[k] = p[(uint64_t)(2 * k + (u ^ 1u)) * it.z + 7];
+                }
+            } else {   // a frame's last block row is among them
+#pragma unroll
+                for (int r = 0; r < 8; r++) {
+                    t[r] = make_uint4(0, 0, 0, 0);
+                    if ((uint32_t)r < ny) {
+                        t[r] = ld16_a4(p + (uint64_t)r * it.z - ((u ^ (uint32_t)r) & 1u));
+                        if ((threadIdx.x & 63u) == 63u) e[r >> 1] = ((u ^ (uint32_t)r) & 1u) ? p[(uint64_t)r * it.z + 7] : e[r >> 1];
+                    }
+                }
             }
 #pragma unroll
             for (int r = 0; r < 8; r++) {
