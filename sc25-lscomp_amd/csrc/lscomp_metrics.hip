@@ -194,51 +194,40 @@ __global__ void copy_tail_kernel(uint8_t *dst, const uint8_t *src, uint32_t n)
 // sum.
 //
 // ALU-bound, so the mapping is chosen for few operations per window.  A lane
-// owns one window column along size0 and kSsimJ windows along size1, and walks
-// planes (size2).  Per row it loads its 8 elements (16 bytes at a dword
-// boundary; neighbouring lanes overlap in L1) and forms the 7-element sums by
-// packed dot products in 32 bits; a plane with a value of 2^14 or more in any
-// of a lane's rows is formed again by 64-bit products.  Along size1, and then
-// along size2, windows overlap by 5 of 7, so a window is the sum of three
-// disjoint pairs and one row (plane); pairs stay in registers, nothing goes
-// through LDS and there is no barrier in the loop.  512 x 1024 x 1024: 1.23 ms
-// against 3.19 ms with one window per thread, double sums through LDS, square
-// roots, divisions and three barriers per plane.  Two windows per lane run at
-// 3 waves per SIMD; with 3 or 4 a plane costs fewer row sums per window but
-// the sums held along size2 leave 2 waves (1.33 and 1.93 ms).
+// owns one word (two elements) of its rows and kSsimJ windows along size1, and
+// walks planes (size2).  It adds its word's values and products over a
+// window's 7 rows, for the pair and for its first element, by packed dot
+// products that accumulate; a window of 7 elements is then three pairs and one
+// element of lanes i .. i + 3, so a wave's 64 words make 61 windows.  Rows 2 to
+// 6 are summed once for both windows.  Along size2 windows overlap by 5 of 7
+// planes, so a window is the sum of three disjoint pairs of planes and one
+// plane; pairs stay in registers, nothing goes through LDS and there is no
+// barrier in the loop.  The next plane's words are loaded before a plane's are
+// used.  512 x 1024 x 1024: 0.77 ms against 1.23 ms with each lane loading and
+// adding the 7 elements of its rows (4.5 rows of 7 elements per window and
+// plane, against 4.5 words), and 3.19 ms with one window per thread, double
+// sums through LDS, square roots, divisions and three barriers per plane;
+// values of 2^14 and more (600 x 1813 x 1558): 2.2, 4.3 and 10.2 ms.  Without
+// the load ahead 0.81 and 2.33 ms.  More windows per lane would leave 2
+// waves per SIMD.
 //
 // Each workgroup writes one partial sum, reduced in a fixed order (here and in
 // ssim_finish_kernel), so the result does not depend on scheduling.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kSsimJ = 2;                            // windows of a lane along size1
-constexpr uint32_t kSsimT0 = 64, kSsimT1 = 4 * kSsimJ;    // windows of a workgroup (4 waves) along size0, size1
+constexpr uint32_t kSsimT0 = 61, kSsimT1 = 4 * kSsimJ;    // windows of a workgroup (4 waves) along size0, size1
 constexpr uint32_t kSsimRows = 2 * kSsimJ + 5;            // rows of a lane's windows
 
-// Sums over 7 elements of one row; extrema still in two halves.
-struct SsimRow {
-    uint32_t sx, sy, mx2, mn2;
-    uint64_t sxy, sqq;   // sums of x y and of x^2 + y^2
-};
 // Sums over a 7 x 7 patch of a plane, and over planes; mm = max | (65535 - min) << 16.
 struct SsimMom {
     uint32_t sx, sy, mm;
     uint64_t sxy, sqq;
 };
 
-__device__ __forceinline__ SsimRow row_add(const SsimRow &a, const SsimRow &b)
-{
-    return {a.sx + b.sx, a.sy + b.sy, pk_max(a.mx2, b.mx2), pk_min(a.mn2, b.mn2), a.sxy + b.sxy, a.sqq + b.sqq};
-}
 __device__ __forceinline__ SsimMom mom_add(const SsimMom &a, const SsimMom &b)
 {
     return {a.sx + b.sx, a.sy + b.sy, pk_max(a.mm, b.mm), a.sxy + b.sxy, a.sqq + b.sqq};
 }
-__device__ __forceinline__ SsimMom mom_of(const SsimRow &r)
-{
-    const uint32_t mx = pk_max(r.mx2, r.mx2 >> 16) & 0xffffu, mn = pk_min(r.mn2, r.mn2 >> 16 | 0xffff0000u) & 0xffffu;
-    return {r.sx, r.sy, mx | (0xffffu - mn) << 16, r.sxy, r.sqq};
-}
-
 __device__ __forceinline__ double ssim_of(const SsimMom &m)
 {
 #pragma clang fp contract(off)
@@ -253,114 +242,145 @@ __device__ __forceinline__ double ssim_of(const SsimMom &m)
     return ((2.0 * pxy + c1) * (2.0 * cov + c2)) / ((pqq + c1) * (var + c2));
 }
 
-// The 7 elements of a lane's row as 4 words: 16 bytes from the dword boundary
-// at or before the first element.  `odd` (uniform): the row's first element is
-// the word's upper half and the last word is whole; else the last word's upper
-// half is an eighth element that does not count.
+// Sums over a lane's word of up to 7 rows: of both elements (p) and of the
+// first one (l).  32 bits hold them (14 products) while every value is below
+// 2^14; kWide: for any value, the products of the first factor's low bytes here
+// and those of its high bytes in h (14 products below 2^24).
+struct SsimProd {
+    uint32_t pxy, pxx, pyy, lxy, lxx, lyy;
+};
 template <bool kWide>
-__device__ __forceinline__ SsimRow ssim_row(u32x4_a4 x, u32x4_a4 y, bool odd, uint32_t &seen)
-{
-    const uint32_t m0 = odd ? 0xffff0000u : 0xffffffffu, m3 = odd ? 0xffffffffu : 0xffffu;
-    const uint32_t lo = x[0] | ~m0, hi = x[3] | ~m3;   // for the minimum
-    x[0] &= m0;
-    y[0] &= m0;
-    x[3] &= m3;
-    y[3] &= m3;
-    SsimRow r;
-    r.mx2 = pk_max(pk_max(x[0], x[1]), pk_max(x[2], x[3]));
-    r.mn2 = pk_min(pk_min(lo, x[1]), pk_min(x[2], hi));
-    r.sx = 0;
-    r.sy = 0;
-    uint32_t xy = 0, qq = 0;
-    r.sxy = 0;
-    r.sqq = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        r.sx = dot2(x[k], 0x00010001u, r.sx);
-        r.sy = dot2(y[k], 0x00010001u, r.sy);
-        if (kWide) {
-            const uint32_t x0 = x[k] & 0xffffu, x1 = x[k] >> 16, y0 = y[k] & 0xffffu, y1 = y[k] >> 16;
-            r.sxy += (uint64_t)(x0 * y0) + (uint64_t)(x1 * y1);
-            r.sqq += (uint64_t)(x0 * x0) + (uint64_t)(x1 * x1) + (uint64_t)(y0 * y0) + (uint64_t)(y1 * y1);
-        } else {   // 14 products below 2^28: 32 bits hold their sum
-            xy = dot2(x[k], y[k], xy);
-            qq = dot2(x[k], x[k], qq);
-            qq = dot2(y[k], y[k], qq);
-        }
-    }
-    if (!kWide) {
-        seen |= x[0] | x[1] | x[2] | x[3] | y[0] | y[1] | y[2] | y[3];
-        r.sxy = xy;
-        r.sqq = qq;
-    }
-    return r;
-}
+struct SsimCol {
+    uint32_t px = 0, py = 0, lx = 0, ly = 0, mx2 = 0, mn2 = 0xffffffffu;
+    SsimProd s{}, h{};
+};
 
-// The 16 bytes of a row by elements, without the one that belongs to no window.
-__device__ __forceinline__ u32x4_a4 ssim_elements(const uint16_t *q, bool odd)
+__device__ __forceinline__ void prod_row(SsimProd &a, uint32_t fx, uint32_t fy, uint32_t x, uint32_t y, uint32_t lx,
+                                         uint32_t ly)
 {
-    uint32_t w0 = 0, w1 = 0, w2 = 0, w3 = 0;
-#pragma unroll 1
-    for (uint32_t k = 0; k < 8; k++) {   // shifted in from above
-        const uint32_t e = (odd ? k != 0 : k != 7) ? q[k] : 0u;
-        w0 = __builtin_amdgcn_alignbit(w1, w0, 16);
-        w1 = __builtin_amdgcn_alignbit(w2, w1, 16);
-        w2 = __builtin_amdgcn_alignbit(w3, w2, 16);
-        w3 = w3 >> 16 | e << 16;
-    }
-    return u32x4_a4{w0, w1, w2, w3};
+    a.pxy = dot2(fx, y, a.pxy);
+    a.pxx = dot2(fx, x, a.pxx);
+    a.pyy = dot2(fy, y, a.pyy);
+    a.lxy = dot2(fx, ly, a.lxy);
+    a.lxx = dot2(fx, lx, a.lxx);
+    a.lyy = dot2(fy, ly, a.lyy);
 }
-
-// The plane sums of a lane's kSsimJ windows: P[j] over rows 2j .. 2j + 6 of the
-// kSsimRows rows from row y0 of the plane that starts at element `plane` (rows
-// past the volume repeat its last one; their windows are not counted).
-// kAny: 64-bit products, and rows by elements when `elements` is set; else
-// 32-bit ones, and the bits seen in any value are returned.
-template <bool kAny>
-__device__ __forceinline__ uint32_t ssim_plane(const uint16_t *ori, const uint16_t *dec, uint64_t plane, uint32_t Y,
-                                               uint32_t Z, uint32_t y0, uint32_t c, uint32_t odd0, bool elements,
-                                               SsimMom P[kSsimJ])
+template <bool kWide>
+__device__ __forceinline__ void col_row(SsimCol<kWide> &a, uint32_t x, uint32_t y)
 {
-    SsimRow even{}, a0{}, a1{}, a2{};   // the last even row, the last three pairs
-    uint32_t seen = 0;
-    const auto step = [&](uint32_t r) -> SsimMom {
-        const uint64_t row = plane + (uint64_t)(y0 + r < Y ? y0 + r : Y - 1u) * Z;
-        const bool odd = (((uint32_t)row ^ odd0) & 1u) != 0;
-        const uint16_t *qx = ori + (row + c - odd), *qy = dec + (row + c - odd);
-        u32x4_a4 x, y;
-        if (kAny && elements) {
-            x = ssim_elements(qx, odd);
-            y = ssim_elements(qy, odd);
-        } else {
-            x = *(const u32x4_a4 *)qx;
-            y = *(const u32x4_a4 *)qy;
-        }
-        const SsimRow v = ssim_row<kAny>(x, y, odd, seen);
-        if (r & 1u) {
-            a0 = a1;
-            a1 = a2;
-            a2 = row_add(even, v);
-            return {};
-        }
-        even = v;
-        return mom_of(row_add(row_add(a0, a1), row_add(a2, v)));
-    };
-    if (kAny) {   // rare: a rolled loop, so that the kernel holds the row's code only once more
-#pragma unroll 1
-        for (uint32_t r = 0; r < kSsimRows; r++) {
-            const SsimMom m = step(r);
-#pragma unroll
-            for (uint32_t j = 0; j < kSsimJ; j++)
-                if (r == 2u * j + 6u) P[j] = m;
-        }
+    const uint32_t lx = x & 0xffffu, ly = y & 0xffffu;
+    a.px = dot2(x, 0x00010001u, a.px);
+    a.py = dot2(y, 0x00010001u, a.py);
+    a.lx += lx;
+    a.ly += ly;
+    a.mx2 = pk_max(a.mx2, x);
+    a.mn2 = pk_min(a.mn2, x);
+    if (kWide) {
+        prod_row(a.s, x & 0x00ff00ffu, y & 0x00ff00ffu, x, y, lx, ly);
+        prod_row(a.h, perm(0u, x, 0x0c030c01u), perm(0u, y, 0x0c030c01u), x, y, lx, ly);
     } else {
-#pragma unroll
-        for (uint32_t r = 0; r < kSsimRows; r++) {
-            const SsimMom m = step(r);
-            if (r >= 6u && (r & 1u) == 0) P[(r - 6u) / 2u] = m;
-        }
+        prod_row(a.s, x, y, x, y, lx, ly);
     }
-    return seen;
+}
+
+// The next lane's value; 0 in lane 63 (wave_shl:1).
+__device__ __forceinline__ uint32_t lane_next(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xf, 0xf, true);
+}
+__device__ __forceinline__ uint64_t lane_next(uint64_t v)
+{
+    return (uint64_t)lane_next((uint32_t)(v >> 32)) << 32 | lane_next((uint32_t)v);
+}
+
+// A lane's window from the columns of lanes i .. i + 3: three whole words and
+// the first element of the last.
+template <bool kWide>
+__device__ __forceinline__ SsimMom col_window(const SsimCol<kWide> &a)
+{
+    const uint32_t nm2 = ~a.mn2;
+    const uint32_t ml = perm(nm2, a.mx2, 0x05040100u), mh = perm(nm2, a.mx2, 0x07060302u);
+    SsimMom w{a.lx, a.ly, ml, a.s.lxy, (uint64_t)a.s.lxx + a.s.lyy};
+    SsimMom p{a.px, a.py, pk_max(ml, mh), a.s.pxy, (uint64_t)a.s.pxx + a.s.pyy};
+    if (kWide) {
+        w.sxy += (uint64_t)a.h.lxy << 8;
+        w.sqq += ((uint64_t)a.h.lxx + a.h.lyy) << 8;
+        p.sxy += (uint64_t)a.h.pxy << 8;
+        p.sqq += ((uint64_t)a.h.pxx + a.h.pyy) << 8;
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        w = mom_add(p, {lane_next(w.sx), lane_next(w.sy), lane_next(w.mm), lane_next(w.sxy), lane_next(w.sqq)});
+    return w;
+}
+
+// A lane's word of each of its rows: elements c and c + 1.  Rows past the
+// volume repeat its last one; their windows are not counted.
+struct SsimWords {
+    uint32_t x[kSsimRows], y[kSsimRows];
+};
+
+// The words from the dword boundary at or before element c of each row.
+template <bool kOdd>
+__device__ __forceinline__ void ssim_load(const uint16_t *ori, const uint16_t *dec, uint64_t plane, uint32_t Y,
+                                          uint32_t Z, uint32_t y0, uint32_t c, uint32_t odd0, SsimWords &w)
+{
+#pragma unroll
+    for (uint32_t r = 0; r < kSsimRows; r++) {
+        const uint64_t row = plane + (uint64_t)(y0 + r < Y ? y0 + r : Y - 1u) * Z;
+        const uint32_t ox = kOdd ? ((uint32_t)row ^ odd0) & 1u : 0u, oy = kOdd ? ((uint32_t)row ^ odd0 >> 1) & 1u : 0u;
+        w.x[r] = *(const uint32_t *)((const uint8_t *)(ori + row - ox) + 2u * c);
+        w.y[r] = *(const uint32_t *)((const uint8_t *)(dec + row - oy) + 2u * c);
+    }
+}
+// Where a word starts one element before c, the second one comes from the next
+// lane's word.
+__device__ __forceinline__ void ssim_shift(uint64_t plane, uint32_t Y, uint32_t Z, uint32_t y0, uint32_t odd0,
+                                           SsimWords &w)
+{
+#pragma unroll
+    for (uint32_t r = 0; r < kSsimRows; r++) {
+        const uint32_t row = (uint32_t)(plane + (uint64_t)(y0 + r < Y ? y0 + r : Y - 1u) * Z);
+        w.x[r] = __builtin_amdgcn_alignbit(lane_next(w.x[r]), w.x[r], 16u * ((row ^ odd0) & 1u));
+        w.y[r] = __builtin_amdgcn_alignbit(lane_next(w.y[r]), w.y[r], 16u * ((row ^ odd0 >> 1) & 1u));
+    }
+}
+// By elements; an element c + 1 past its row is never used.  Rare, so a rolled
+// loop that shifts the words into place: unrolled, its loads cost the kernel 45
+// spilled registers.
+__device__ __forceinline__ void ssim_words_by_element(const uint16_t *ori, const uint16_t *dec, uint64_t plane,
+                                                      uint32_t Y, uint32_t Z, uint32_t y0, uint32_t c, SsimWords &w)
+{
+    const uint32_t c1 = c + 1u < Z ? c + 1u : Z - 1u;
+    w = {};
+#pragma unroll 1
+    for (uint32_t r = 0; r < kSsimRows; r++) {
+        const uint64_t row = plane + (uint64_t)(y0 + r < Y ? y0 + r : Y - 1u) * Z;
+#pragma unroll
+        for (uint32_t k = 0; k + 1 < kSsimRows; k++) {
+            w.x[k] = w.x[k + 1];
+            w.y[k] = w.y[k + 1];
+        }
+        w.x[kSsimRows - 1] = ori[row + c] | (uint32_t)ori[row + c1] << 16;
+        w.y[kSsimRows - 1] = dec[row + c] | (uint32_t)dec[row + c1] << 16;
+    }
+}
+
+// The plane sums of a lane's kSsimJ windows: P[j] over rows 2j .. 2j + 6.
+template <bool kWide>
+__device__ __forceinline__ void ssim_plane(const SsimWords &w, SsimMom P[kSsimJ])
+{
+    static_assert(kSsimJ == 2, "rows 2 .. 6 are those of both windows");
+    SsimCol<kWide> b;
+#pragma unroll
+    for (uint32_t r = 2; r < 7; r++) col_row(b, w.x[r], w.y[r]);
+    SsimCol<kWide> a = b;
+    col_row(a, w.x[0], w.y[0]);
+    col_row(a, w.x[1], w.y[1]);
+    P[0] = col_window(a);
+    col_row(b, w.x[7], w.y[7]);
+    col_row(b, w.x[8], w.y[8]);
+    P[1] = col_window(b);
 }
 
 // One workgroup per (size0 tile, size1 tile, size2 chunk) of windows; grid nb0
@@ -379,8 +399,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     const uint32_t b1 = blk % nb1, b2 = blk / nb1;
     const uint32_t o0 = b0 * kSsimT0 + lane, o1 = b1 * kSsimT1 + wave * kSsimJ, o2 = b2 * chunk;
     const uint32_t nw = n2 - o2 < chunk ? n2 - o2 : chunk;   // windows along size2
-    const uint32_t c = 2u * (o0 < n0 ? o0 : n0 - 1u);        // first element of the window's rows
-    const bool mixed = odd0 == 1u || odd0 == 2u;             // the volumes' rows differ in alignment
+    // a lane's word: that of its window, and for the last windows the three words after them
+    const uint32_t c = 2u * (o0 < n0 + 2u ? o0 : n0 + 2u);
+    const bool odd = (Z & 1u) || odd0;
     double acc = 0.0;
     if (o1 < n1) {
         // carry: after an odd plane the last three pairs of planes, after an
@@ -388,17 +409,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         SsimMom carry[kSsimJ] = {}, s2[kSsimJ] = {}, s1[kSsimJ] = {};
         const uint64_t per_plane = (uint64_t)Y * Z;
         uint64_t plane = 2ull * o2 * per_plane;
+        const uint64_t last = (X - 1u) * per_plane;
+        // a word can leave a volume, by one element, only in its first row (a
+        // base at 2 mod 4) and in its last: the first or last plane by
+        // elements; its neighbour is loaded in its place
+        const bool edge0 = o1 == 0 && odd0, edge1 = 2u * o1 + kSsimRows >= Y;
+        const auto safe = [&](uint64_t p) -> uint64_t {
+            if (p >= last) return edge1 ? last - per_plane : last;
+            return p == 0 && edge0 ? per_plane : p;
+        };
+        SsimWords next;
+        if (odd)
+            ssim_load<true>(ori, dec, safe(plane), Y, Z, 2u * o1, c, odd0, next);
+        else
+            ssim_load<false>(ori, dec, safe(plane), Y, Z, 2u * o1, c, odd0, next);
         // planes 2 o2 .. 2 o2 + 2 nw + 4, the last one at most X - 1
         for (uint32_t i = 0; i < 2u * nw + 5u; i++, plane += per_plane) {
             SsimMom P[kSsimJ];
-            // a row's 16 bytes can leave a volume, by one element, only in its
-            // first row (a base at 2 mod 4) and in its last
-            const bool elements = mixed || (plane == 0 && o1 == 0 && odd0) ||
-                                  (plane == (X - 1u) * per_plane && 2u * o1 + kSsimRows >= Y);
-            uint32_t seen = 0xffffffffu;
-            if (!elements) seen = ssim_plane<false>(ori, dec, plane, Y, Z, 2u * o1, c, odd0, false, P);
+            SsimWords w = next;
+            if (i == 2u * nw + 4u)
+                ;
+            else if (odd)
+                ssim_load<true>(ori, dec, safe(plane + per_plane), Y, Z, 2u * o1, c, odd0, next);
+            else
+                ssim_load<false>(ori, dec, safe(plane + per_plane), Y, Z, 2u * o1, c, odd0, next);
+            if ((plane == 0 && edge0) || (plane == last && edge1))
+                ssim_words_by_element(ori, dec, plane, Y, Z, 2u * o1, c, w);
+            else if (odd)
+                ssim_shift(plane, Y, Z, 2u * o1, odd0, w);
+            uint32_t seen = 0;
+#pragma unroll
+            for (uint32_t r = 0; r < kSsimRows; r++) seen |= w.x[r] | w.y[r];
             if (__ballot((seen & 0xc000c000u) != 0))
-                ssim_plane<true>(ori, dec, plane, Y, Z, 2u * o1, c, odd0, elements, P);
+                ssim_plane<true>(w, P);
+            else
+                ssim_plane<false>(w, P);
             if (i & 1u) {
 #pragma unroll
                 for (uint32_t j = 0; j < kSsimJ; j++) {
@@ -412,7 +457,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 #pragma unroll
                     for (uint32_t j = 0; j < kSsimJ; j++) {
                         const double s = ssim_of(mom_add(carry[j], P[j]));
-                        acc += o0 < n0 && o1 + j < n1 ? s : 0.0;
+                        acc += lane < kSsimT0 && o0 < n0 && o1 + j < n1 ? s : 0.0;
                     }
                 }
 #pragma unroll
@@ -517,12 +562,15 @@ extern "C" int lscomp_ssim_u16(const uint16_t *d_orig, const uint16_t *d_dec, ls
     if (dims.x < 7 || dims.y < 7 || dims.z < 7) return LSCOMP_ERR_INVALID_ARG;   // no window fits
     const uint32_t n0 = (dims.z - 7) / 2 + 1, n1 = (dims.y - 7) / 2 + 1, n2 = (dims.x - 7) / 2 + 1;
     const uint32_t nb0 = (n0 + kSsimT0 - 1) / kSsimT0, nb1 = (n1 + kSsimT1 - 1) / kSsimT1;
-    // windows of a workgroup along size2: a chunk of k reads 2 k + 5 planes, so
-    // 32 where the volume gives enough workgroups (3 waves per SIMD run at
-    // once), fewer for small volumes
-    uint32_t chunk = 32;
-    while (chunk > 4 && (uint64_t)nb0 * nb1 * ((n2 + chunk - 1) / chunk) < 2048) chunk /= 2;
-    const uint32_t nc = (n2 + chunk - 1) / chunk;
+    // A chunk of k windows along size2 reads 2 k + 5 planes, so as few chunks as
+    // fill the chip once (256 CUs hold 3 workgroups each), of 4 to 32 windows:
+    // 205 x 553 x 256 99 us in 735 workgroups, 117 in 2625; 100 x 512 x 512 80
+    // us in 640, 91 in 2560; 60 x 1813 x 1558 249 us in 1469, 284 in 5876.
+    // From 32 up a chunk gains nothing (512 x 1024 x 1024: 755 us at 64, 765).
+    const uint64_t fill = 768 / ((uint64_t)nb0 * nb1);
+    const uint32_t most = (n2 + 3) / 4, least = (n2 + 31) / 32;
+    const uint32_t want = fill < least ? least : fill > most ? most : (uint32_t)fill;
+    const uint32_t chunk = (n2 + want - 1) / want, nc = (n2 + chunk - 1) / chunk;
     const uint64_t blocks = (uint64_t)nb0 * nb1 * nc;
     if (blocks > 0x7fffffffull) return LSCOMP_ERR_TOO_LARGE;
     AuxLease aux(stream, (blocks + 1) * sizeof(double), sizeof(double));

@@ -179,3 +179,19 @@ def test_ssim_rejects_volumes_without_a_window(gpu):
     v = _dev(np.zeros((6, 10, 10), np.uint16))
     with pytest.raises(lscomp.LscompError):
         gpu.ssim(v, v, (6, 10, 10))
+
+
+# a wave's 61 windows along size0 and the ones around them (61 fit in 127 and 128
+# elements), the first elements of a window in the wave's last words; one to four
+# chunks along size2; products in 32 bits from values on both sides of a byte,
+# of 2^14 and of 2^16
+@pytest.mark.parametrize("shape", [(7, 9, 126), (8, 9, 127), (7, 10, 128), (9, 8, 129), (7, 9, 130), (7, 23, 251),
+                                   (45, 9, 131)], ids=lambda s: "x".join(map(str, s)))
+def test_ssim_wave_edges_and_products(gpu, orc, shape):
+    rng = np.random.default_rng(sum(shape))
+    for top in (2, 1 << 8, 1 << 14, 1 << 16):
+        a = rng.integers(0, top, shape).astype(np.uint16)
+        b = rng.integers(0, top, shape).astype(np.uint16)
+        for x, y in ((a, b), (np.full_like(a, top - 1), b), (a, a)):
+            got, want = gpu.ssim(_dev(x), _dev(y), shape), orc.ssim(x, y)
+            assert got == pytest.approx(want, rel=1e-10, abs=1e-13), top
