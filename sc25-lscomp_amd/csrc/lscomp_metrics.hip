@@ -203,13 +203,14 @@ __global__ void copy_tail_kernel(uint8_t *dst, const uint8_t *src, uint32_t n)
 // planes, so a window is the sum of three disjoint pairs of planes and one
 // plane; pairs stay in registers, nothing goes through LDS and there is no
 // barrier in the loop.  The next plane's words are loaded before a plane's are
-// used.  512 x 1024 x 1024: 0.77 ms against 1.23 ms with each lane loading and
-// adding the 7 elements of its rows (4.5 rows of 7 elements per window and
-// plane, against 4.5 words), and 3.19 ms with one window per thread, double
-// sums through LDS, square roots, divisions and three barriers per plane;
-// values of 2^14 and more (600 x 1813 x 1558): 2.2, 4.3 and 10.2 ms.  Without
-// the load ahead 0.81 and 2.33 ms.  More windows per lane would leave 2
-// waves per SIMD.
+// used.  512 x 1024 x 1024 (values below 2^12): 0.66 ms, against 1.23 ms with
+// each lane loading and adding the 7 elements of its rows (4.5 rows of 7
+// elements per window and plane, against 4.5 words), and 3.19 ms with one
+// window per thread, double sums through LDS, square roots, divisions and three
+// barriers per plane; 600 x 1813 x 1558 with 16-bit values 2.1, 4.3 and 10.2
+// ms.  Without the narrow sums' packed halves and 32-bit window products 0.77
+// ms, without the load ahead 4 % more; 4 waves per SIMD (128 registers) 0.72
+// and 2.36 ms.  The vector ALU is busy all the time.
 //
 // Each workgroup writes one partial sum, reduced in a fixed order (here and in
 // ssim_finish_kernel), so the result does not depend on scheduling.
@@ -243,30 +244,50 @@ __device__ __forceinline__ double ssim_of(const SsimMom &m)
 }
 
 // Sums over a lane's word of up to 7 rows: of both elements (p) and of the
-// first one (l).  32 bits hold them (14 products) while every value is below
-// 2^14; kWide: for any value, the products of the first factor's low bytes here
-// and those of its high bytes in h (14 products below 2^24).
-struct SsimProd {
-    uint32_t pxy, pxx, pyy, lxy, lxx, lyy;
-};
-template <bool kWide>
+// first one (l).  Narrow, every value below 2^12: the values' sums in packed
+// halves (7 values), and the products of a window's 49 elements fit 32 bits,
+// those of x^2 + y^2 too.
 struct SsimCol {
+    uint32_t sx2 = 0, sy2 = 0, mx2 = 0, mn2 = 0xffffffffu, pxy = 0, pqq = 0, lxy = 0, lqq = 0;
+};
+// Any value: the products of the first factor's low bytes in s and those of its
+// high bytes in h; 98 products below 2^24 fit 32 bits.
+struct SsimProd {
+    uint32_t pxy, pqq, lxy, lqq;
+};
+struct SsimColWide {
     uint32_t px = 0, py = 0, lx = 0, ly = 0, mx2 = 0, mn2 = 0xffffffffu;
     SsimProd s{}, h{};
 };
 
+// The product of the low halves, added to c; written out because the compiler
+// takes two masks, a 24-bit product and an addition for it.
+__device__ __forceinline__ uint32_t mad_low(uint32_t a, uint32_t b, uint32_t c)
+{
+    uint32_t r;
+    asm("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ void col_row(SsimCol &a, uint32_t x, uint32_t y)
+{
+    a.sx2 = as_u32(as_u16x2(a.sx2) + as_u16x2(x));
+    a.sy2 = as_u32(as_u16x2(a.sy2) + as_u16x2(y));
+    a.mx2 = pk_max(a.mx2, x);
+    a.mn2 = pk_min(a.mn2, x);
+    a.pxy = dot2(x, y, a.pxy);
+    a.pqq = dot2(y, y, dot2(x, x, a.pqq));
+    a.lxy = mad_low(x, y, a.lxy);
+    a.lqq = mad_low(y, y, mad_low(x, x, a.lqq));
+}
 __device__ __forceinline__ void prod_row(SsimProd &a, uint32_t fx, uint32_t fy, uint32_t x, uint32_t y, uint32_t lx,
                                          uint32_t ly)
 {
     a.pxy = dot2(fx, y, a.pxy);
-    a.pxx = dot2(fx, x, a.pxx);
-    a.pyy = dot2(fy, y, a.pyy);
+    a.pqq = dot2(fy, y, dot2(fx, x, a.pqq));
     a.lxy = dot2(fx, ly, a.lxy);
-    a.lxx = dot2(fx, lx, a.lxx);
-    a.lyy = dot2(fy, ly, a.lyy);
+    a.lqq = dot2(fy, ly, dot2(fx, lx, a.lqq));
 }
-template <bool kWide>
-__device__ __forceinline__ void col_row(SsimCol<kWide> &a, uint32_t x, uint32_t y)
+__device__ __forceinline__ void col_row(SsimColWide &a, uint32_t x, uint32_t y)
 {
     const uint32_t lx = x & 0xffffu, ly = y & 0xffffu;
     a.px = dot2(x, 0x00010001u, a.px);
@@ -275,12 +296,8 @@ __device__ __forceinline__ void col_row(SsimCol<kWide> &a, uint32_t x, uint32_t 
     a.ly += ly;
     a.mx2 = pk_max(a.mx2, x);
     a.mn2 = pk_min(a.mn2, x);
-    if (kWide) {
-        prod_row(a.s, x & 0x00ff00ffu, y & 0x00ff00ffu, x, y, lx, ly);
-        prod_row(a.h, perm(0u, x, 0x0c030c01u), perm(0u, y, 0x0c030c01u), x, y, lx, ly);
-    } else {
-        prod_row(a.s, x, y, x, y, lx, ly);
-    }
+    prod_row(a.s, x & 0x00ff00ffu, y & 0x00ff00ffu, x, y, lx, ly);
+    prod_row(a.h, perm(0u, x, 0x0c030c01u), perm(0u, y, 0x0c030c01u), x, y, lx, ly);
 }
 
 // The next lane's value; 0 in lane 63 (wave_shl:1).
@@ -288,30 +305,40 @@ __device__ __forceinline__ uint32_t lane_next(uint32_t v)
 {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xf, 0xf, true);
 }
-__device__ __forceinline__ uint64_t lane_next(uint64_t v)
-{
-    return (uint64_t)lane_next((uint32_t)(v >> 32)) << 32 | lane_next((uint32_t)v);
-}
-
 // A lane's window from the columns of lanes i .. i + 3: three whole words and
 // the first element of the last.
-template <bool kWide>
-__device__ __forceinline__ SsimMom col_window(const SsimCol<kWide> &a)
+__device__ __forceinline__ SsimMom col_window(const SsimCol &a)
 {
     const uint32_t nm2 = ~a.mn2;
-    const uint32_t ml = perm(nm2, a.mx2, 0x05040100u), mh = perm(nm2, a.mx2, 0x07060302u);
-    SsimMom w{a.lx, a.ly, ml, a.s.lxy, (uint64_t)a.s.lxx + a.s.lyy};
-    SsimMom p{a.px, a.py, pk_max(ml, mh), a.s.pxy, (uint64_t)a.s.pxx + a.s.pyy};
-    if (kWide) {
-        w.sxy += (uint64_t)a.h.lxy << 8;
-        w.sqq += ((uint64_t)a.h.lxx + a.h.lyy) << 8;
-        p.sxy += (uint64_t)a.h.pxy << 8;
-        p.sqq += ((uint64_t)a.h.pxx + a.h.pyy) << 8;
-    }
+    const uint32_t ml = perm(nm2, a.mx2, 0x05040100u), mp = pk_max(ml, perm(nm2, a.mx2, 0x07060302u));
+    const uint32_t lx = a.sx2 & 0xffffu, ly = a.sy2 & 0xffffu, px = lx + (a.sx2 >> 16), py = ly + (a.sy2 >> 16);
+    uint32_t sx = lx, sy = ly, mm = ml, xy = a.lxy, qq = a.lqq;
 #pragma unroll
-    for (int k = 0; k < 3; k++)
-        w = mom_add(p, {lane_next(w.sx), lane_next(w.sy), lane_next(w.mm), lane_next(w.sxy), lane_next(w.sqq)});
-    return w;
+    for (int k = 0; k < 3; k++) {
+        sx = px + lane_next(sx);
+        sy = py + lane_next(sy);
+        mm = pk_max(mp, lane_next(mm));
+        xy = a.pxy + lane_next(xy);
+        qq = a.pqq + lane_next(qq);
+    }
+    return {sx, sy, mm, xy, qq};
+}
+__device__ __forceinline__ SsimMom col_window(const SsimColWide &a)
+{
+    const uint32_t nm2 = ~a.mn2;
+    const uint32_t ml = perm(nm2, a.mx2, 0x05040100u), mp = pk_max(ml, perm(nm2, a.mx2, 0x07060302u));
+    uint32_t sx = a.lx, sy = a.ly, mm = ml, xys = a.s.lxy, xyh = a.h.lxy, qqs = a.s.lqq, qqh = a.h.lqq;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        sx = a.px + lane_next(sx);
+        sy = a.py + lane_next(sy);
+        mm = pk_max(mp, lane_next(mm));
+        xys = a.s.pxy + lane_next(xys);
+        xyh = a.h.pxy + lane_next(xyh);
+        qqs = a.s.pqq + lane_next(qqs);
+        qqh = a.h.pqq + lane_next(qqh);
+    }
+    return {sx, sy, mm, ((uint64_t)xyh << 8) + xys, ((uint64_t)qqh << 8) + qqs};
 }
 
 // A lane's word of each of its rows: elements c and c + 1.  Rows past the
@@ -320,17 +347,25 @@ struct SsimWords {
     uint32_t x[kSsimRows], y[kSsimRows];
 };
 
+typedef const __attribute__((address_space(1))) uint8_t *GlobalBytes;
+
 // The words from the dword boundary at or before element c of each row.
 template <bool kOdd>
 __device__ __forceinline__ void ssim_load(const uint16_t *ori, const uint16_t *dec, uint64_t plane, uint32_t Y,
                                           uint32_t Z, uint32_t y0, uint32_t c, uint32_t odd0, SsimWords &w)
 {
+    uint32_t at = 2u * c;
+    asm("" : "+v"(at));   // keeps the zero extension beside the loads, which take it as their offset
 #pragma unroll
     for (uint32_t r = 0; r < kSsimRows; r++) {
         const uint64_t row = plane + (uint64_t)(y0 + r < Y ? y0 + r : Y - 1u) * Z;
         const uint32_t ox = kOdd ? ((uint32_t)row ^ odd0) & 1u : 0u, oy = kOdd ? ((uint32_t)row ^ odd0 >> 1) & 1u : 0u;
-        w.x[r] = *(const uint32_t *)((const uint8_t *)(ori + row - ox) + 2u * c);
-        w.y[r] = *(const uint32_t *)((const uint8_t *)(dec + row - oy) + 2u * c);
+        // the row in scalar registers plus the lane's offset, not a 64-bit vector add per row
+        GlobalBytes qx = (GlobalBytes)(ori + row - ox), qy = (GlobalBytes)(dec + row - oy);
+        asm("" : "+s"(qx));
+        asm("" : "+s"(qy));
+        w.x[r] = *(const __attribute__((address_space(1))) uint32_t *)(qx + at);
+        w.y[r] = *(const __attribute__((address_space(1))) uint32_t *)(qy + at);
     }
 }
 // Where a word starts one element before c, the second one comes from the next
@@ -367,14 +402,14 @@ __device__ __forceinline__ void ssim_words_by_element(const uint16_t *ori, const
 }
 
 // The plane sums of a lane's kSsimJ windows: P[j] over rows 2j .. 2j + 6.
-template <bool kWide>
+template <class Col>
 __device__ __forceinline__ void ssim_plane(const SsimWords &w, SsimMom P[kSsimJ])
 {
     static_assert(kSsimJ == 2, "rows 2 .. 6 are those of both windows");
-    SsimCol<kWide> b;
+    Col b;
 #pragma unroll
     for (uint32_t r = 2; r < 7; r++) col_row(b, w.x[r], w.y[r]);
-    SsimCol<kWide> a = b;
+    Col a = b;
     col_row(a, w.x[0], w.y[0]);
     col_row(a, w.x[1], w.y[1]);
     P[0] = col_window(a);
@@ -440,10 +475,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
             uint32_t seen = 0;
 #pragma unroll
             for (uint32_t r = 0; r < kSsimRows; r++) seen |= w.x[r] | w.y[r];
-            if (__ballot((seen & 0xc000c000u) != 0))
-                ssim_plane<true>(w, P);
+            if (__ballot((seen & 0xf000f000u) != 0))
+                ssim_plane<SsimColWide>(w, P);
             else
-                ssim_plane<false>(w, P);
+                ssim_plane<SsimCol>(w, P);
             if (i & 1u) {
 #pragma unroll
                 for (uint32_t j = 0; j < kSsimJ; j++) {
@@ -564,9 +599,10 @@ extern "C" int lscomp_ssim_u16(const uint16_t *d_orig, const uint16_t *d_dec, ls
     const uint32_t nb0 = (n0 + kSsimT0 - 1) / kSsimT0, nb1 = (n1 + kSsimT1 - 1) / kSsimT1;
     // A chunk of k windows along size2 reads 2 k + 5 planes, so as few chunks as
     // fill the chip once (256 CUs hold 3 workgroups each), of 4 to 32 windows:
-    // 205 x 553 x 256 99 us in 735 workgroups, 117 in 2625; 100 x 512 x 512 80
-    // us in 640, 91 in 2560; 60 x 1813 x 1558 249 us in 1469, 284 in 5876.
-    // From 32 up a chunk gains nothing (512 x 1024 x 1024: 755 us at 64, 765).
+    // 205 x 553 x 256 89 us in 735 workgroups, 104 in 2625; 100 x 512 x 512 68
+    // us in 640, 77 in 2560; 60 x 1813 x 1558 227 us in 1469, 254 in 5876.
+    // Longer chunks gain nothing (512 x 1024 x 1024: 653 us at 32, 641 at 40,
+    // 684 at 64).
     const uint64_t fill = 768 / ((uint64_t)nb0 * nb1);
     const uint32_t most = (n2 + 3) / 4, least = (n2 + 31) / 32;
     const uint32_t want = fill < least ? least : fill > most ? most : (uint32_t)fill;

@@ -183,13 +183,13 @@ def test_ssim_rejects_volumes_without_a_window(gpu):
 
 # a wave's 61 windows along size0 and the ones around them (61 fit in 127 and 128
 # elements), the first elements of a window in the wave's last words; one to four
-# chunks along size2; products in 32 bits from values on both sides of a byte,
-# of 2^14 and of 2^16
+# chunks along size2; sums in 32 bits at their largest: values of one byte, of 12
+# bits (the narrow sums' limit), of 14 and of 16
 @pytest.mark.parametrize("shape", [(7, 9, 126), (8, 9, 127), (7, 10, 128), (9, 8, 129), (7, 9, 130), (7, 23, 251),
                                    (45, 9, 131)], ids=lambda s: "x".join(map(str, s)))
 def test_ssim_wave_edges_and_products(gpu, orc, shape):
     rng = np.random.default_rng(sum(shape))
-    for top in (2, 1 << 8, 1 << 14, 1 << 16):
+    for top in (2, 1 << 8, 1 << 12, 1 << 14, 1 << 16):
         a = rng.integers(0, top, shape).astype(np.uint16)
         b = rng.integers(0, top, shape).astype(np.uint16)
         for x, y in ((a, b), (np.full_like(a, top - 1), b), (a, a)):
