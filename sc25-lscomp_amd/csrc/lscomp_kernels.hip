@@ -895,10 +895,11 @@ __device__ __forceinline__ void finish_launch(Ctrl *ctrl, uint32_t epoch)
 {
     __syncthreads();
     if (threadIdx.x == 0) {
-        // a time-out of a look-back is flagged by this thread, so it is seen here
-        if (__hip_atomic_load(&ctrl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERRF_TIMEOUT)
-            flag_error(ctrl, ERRF_TIMEOUT);
+        // a time-out of a look-back is flagged by this thread, so it is seen here;
+        // looked at after the count, so that both round trips run together
+        const uint32_t err = __hip_atomic_load(&ctrl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         count_done(ctrl, epoch, gridDim.x);
+        if (err & ERRF_TIMEOUT) flag_error(ctrl, ERRF_TIMEOUT);
     }
 }
 
