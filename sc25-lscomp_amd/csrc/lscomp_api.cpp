@@ -171,7 +171,6 @@ struct Scratch {
     uint64_t *tile_off = nullptr;  // device, cap_tiles + 1 decode tile offsets
     uint64_t launches = 0;         // epochs used since the status words were cleared
     CtrlHost *host = nullptr;      // pinned, written by the kernels
-    bool copy_head = false;        // a uint32 compression ran since the last wait_host
     void *aux = nullptr;           // device, kAuxKeep bytes (AuxLease), allocated at first use
     std::mutex mu;
 };
@@ -250,12 +249,6 @@ int count_launch(Scratch *s)
 // Waits for the stream; s->host then holds what its launches left.
 int wait_host(Scratch *s)
 {
-    if (s->copy_head) {
-        const int st = hip_fail(hipMemcpyAsync(s->host, s->ctrl, kCtrlHead, hipMemcpyDeviceToHost, s->stream),
-                                "hipMemcpyAsync");
-        if (st) return st;
-        s->copy_head = false;
-    }
     return hip_fail(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
 }
 
@@ -263,7 +256,7 @@ int wait_host(Scratch *s)
 int take_errors(Scratch *s)
 {
     volatile uint32_t *f = s->host->flags;
-    const uint32_t e = s->host->error | (f[0] ? 1u : 0u) | (f[1] ? 2u : 0u);
+    const uint32_t e = (f[0] ? 1u : 0u) | (f[1] ? 2u : 0u) | (f[2] ? 4u : 0u);
     static_assert(ERRF_CORRUPT == 1u && ERRF_TIMEOUT == 2u && ERRF_RANGE == 4u, "flag words by bit");
     if (!e) return LSCOMP_OK;
     int st = hip_fail(launch_fill_u64((uint64_t *)&s->ctrl->error, 1, 0, s->stream), "fill");
@@ -271,7 +264,6 @@ int take_errors(Scratch *s)
     st = hip_fail(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
     if (st) return st;
     f[0] = f[1] = f[2] = 0;
-    s->host->error = 0;
     if (e & ERRF_TIMEOUT) return LSCOMP_ERR_INTERNAL;
     if (e & ERRF_RANGE) return LSCOMP_ERR_RANGE;
     return LSCOMP_ERR_CORRUPT;
@@ -397,8 +389,7 @@ int launch_item_u32(Scratch *s, Item &it, bool compress)
     cfg.sched.nc = nc < cfg.grid ? (nc ? nc : 1u) : cfg.grid;
     cfg.sched.win = default_window(cfg.tile);
     if (compress) {
-        if (!it.result) it.result = &s->ctrl->result;
-        s->copy_head = true;
+        if (!it.result) it.result = &s->host->size;
     } else {
         cfg.tile_off = s->tile_off;
         cfg.off_mode = g_decode_mode.load() == 2 ? OFF_KERNEL : OFF_PHASE;
@@ -561,7 +552,7 @@ int lscomp_compress_u32(const uint32_t *d_in, uint8_t *d_out, size_t out_capacit
     if (st) return st;
     st = wait_host(s);
     if (st) return st;
-    *out_bytes = (size_t)*(volatile uint64_t *)&s->host->result;
+    *out_bytes = (size_t)*(volatile uint64_t *)&s->host->size;
     st = take_errors(s);
     if (st) return st;
     return *out_bytes > out_capacity ? LSCOMP_ERR_CAPACITY : LSCOMP_OK;

@@ -38,9 +38,8 @@ struct CtrLine {
 struct Ctrl {
     uint32_t error;      // sticky ERRF_* bits, cleared by the host
     uint32_t pad2;
-    uint64_t result;     // stream bytes of a blocking uint32 compression
     uint32_t *flags;     // host-pinned: word k is set with bit k of error (null: none)
-    uint64_t pad3[13];
+    uint64_t pad3[14];
     uint32_t done_ctr;   // workgroups finished
     uint32_t epoch;      // tags look-back words of the current launch (read once per workgroup)
     uint32_t pad1[30];
@@ -50,19 +49,16 @@ struct Ctrl {
     CtrLine ctr[kMaxCounters];   // tile ids, one counter per class
 };
 static_assert(sizeof(Ctrl) == 768 + 256 * kMaxCounters, "Ctrl layout");
-constexpr size_t kCtrlHead = 16;   // error and result: what the host copies after a uint32 compression
 // What a launch leaves for the host of a single-volume call, in pinned memory.
-// The kernels write the flags and a blocking uint16 compression's size there
-// themselves: the copy of the control head took a blocking call 2-3 us (512 x
-// 512 compression 24.0 -> 22.1 us, 16 x 512 x 512 decompression 25.5 -> 23.6).
-// After a uint32 compression, which can set ERRF_RANGE, the head is copied.
+// The kernels write every error flag and a blocking compression's size there
+// themselves, so that the host finds them after any launch of the stream, a
+// replayed one too, and copies nothing: the copy of the control head took a
+// blocking call 2-3 us (512 x 512 compression 24.0 -> 22.1 us, 16 x 512 x 512
+// decompression 25.5 -> 23.6).
 struct CtrlHost {
-    uint32_t error;      // copied head
-    uint32_t pad0;
-    uint64_t result;
-    uint64_t size;       // stream bytes of the last blocking uint16 compression
-    uint32_t flags[3];   // word k: bit k of Ctrl::error has been set (sticky; all but ERRF_RANGE)
-    uint32_t pad1[55];
+    uint64_t size;       // stream bytes of the last blocking compression
+    uint32_t flags[3];   // word k: bit k of Ctrl::error has been set (sticky)
+    uint32_t pad1[59];
     uint8_t aux[1024];   // AuxLease results
 };
 static_assert(sizeof(CtrlHost) == 256 + 1024, "CtrlHost layout");

@@ -71,14 +71,23 @@ __device__ __forceinline__ void st_relaxed(uint64_t *p, uint64_t v)
 }
 
 // Flags the launch (one ERRF_* bit), also where the host reads without a copy.
-// Not for the hot loops of compression, which set Ctrl::error alone (this code
-// in the look-back took uint32 compression 740 -> 745 us): finish_launch
-// passes a time-out on, and the host copies the word for ERRF_RANGE.
+// Not for the hot loops of compression (this code in the look-back took uint32
+// compression 740 -> 745 us): those set a bit of launch_flags, which
+// finish_launch passes on.
 __device__ __forceinline__ void flag_error(Ctrl *ctrl, uint32_t bit)
 {
     __hip_atomic_fetch_or(&ctrl->error, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     uint32_t *h = ctrl->flags;
     if (h) __hip_atomic_store(h + __builtin_ctz(bit), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// ERRF_* bits a workgroup of a persistent launch has met, in LDS: any thread
+// sets one, thread 0 clears them before the first barrier, and finish_launch
+// flags the launch with them.
+__device__ __forceinline__ uint32_t &launch_flags()
+{
+    __shared__ uint32_t flags;
+    return flags;
 }
 
 // Inclusive scan over the wave's 64 lanes with DPP moves: shifts by 1, 2, 4 and
@@ -540,7 +549,7 @@ struct CodecU16T {
     {
         load_block<kRows>(it, bx, by, bz, R);
     }
-    __device__ __forceinline__ static uint32_t header(const uint32_t R[kRegs], const Item &it, Ctrl *)
+    __device__ __forceinline__ static uint32_t header(const uint32_t R[kRegs], const Item &it, bool &)
     {
         return block_header<kMem, kKind>(R, it.dec);
     }
@@ -569,17 +578,12 @@ struct CodecU32 {
         load_block_u32(it, bx, by, bz, R);
     }
     // A block whose quantized maximum needs 32 bits is not representable: the
-    // launch is flagged and the block's rate cleared, so the stream stays
-    // consistent.
-    __device__ __forceinline__ static uint32_t header(const uint32_t R[kRegs], const Item &it, Ctrl *ctrl)
+    // caller flags the launch (rate32), and the block's rate is cleared, so the
+    // stream stays consistent.
+    __device__ __forceinline__ static uint32_t header(const uint32_t R[kRegs], const Item &it, bool &rate32)
     {
-        bool rate32 = false;
-        uint32_t hdr = block_header_u32(R, it.dec, &rate32);
-        if (rate32) {
-            __hip_atomic_fetch_or(&ctrl->error, ERRF_RANGE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            hdr &= 0xe0u;
-        }
-        return hdr;
+        const uint32_t hdr = block_header_u32(R, it.dec, &rate32);
+        return rate32 ? hdr & 0xe0u : hdr;
     }
     __device__ __forceinline__ static void encode(uint32_t R[kRegs], uint32_t hdr, const Item &it, uint32_t *out)
     {
@@ -900,6 +904,7 @@ __device__ __forceinline__ void finish_launch(Ctrl *ctrl, uint32_t epoch)
         const uint32_t err = __hip_atomic_load(&ctrl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         count_done(ctrl, epoch, gridDim.x);
         if (err & ERRF_TIMEOUT) flag_error(ctrl, ERRF_TIMEOUT);
+        if (launch_flags() & ERRF_RANGE) flag_error(ctrl, ERRF_RANGE);
     }
 }
 
@@ -1100,6 +1105,7 @@ __device__ __forceinline__ void compress_tiles(const Item single, const Item *__
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t win = sc.win;
     if (tid == 0) {
+        launch_flags() = 0;
         sh.epoch = __hip_atomic_load(&ctrl->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         sh.ntot = d_total_tiles ? *d_total_tiles : total_tiles;
         // the first tile: with one counter its first value, with several the
@@ -1152,7 +1158,9 @@ __device__ __forceinline__ void compress_tiles(const Item single, const Item *__
         uint32_t n_hdr = 0, n_words = 0;
         if (have_n) {
             if (nvalid) {
-                n_hdr = C::header(D, item_at<kTable>(single, items, n_item), ctrl);
+                bool rate32 = false;
+                n_hdr = C::header(D, item_at<kTable>(single, items, n_item), rate32);
+                if (rate32) atomicOr(&launch_flags(), ERRF_RANGE);
                 n_words = header_payload_bytes(n_hdr) >> 2;
             }
             ((uint8_t *)sh.hdr[hb])[tid] = (uint8_t)n_hdr;
@@ -1279,7 +1287,9 @@ __device__ __forceinline__ void compress_small_tile(const Item &it, Ctrl *ctrl, 
             uint32_t bx, by, bz;
             block_coords(it, b, bx, by, bz);
             C::load(it, bx, by, bz, D);
-            hdr = C::header(D, it, ctrl);
+            bool rate32 = false;
+            hdr = C::header(D, it, rate32);
+            if (rate32) flag_error(ctrl, ERRF_RANGE);
         }
         return header_payload_bytes(hdr) >> 2;
     };
@@ -1526,6 +1536,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void 
     __shared__ TileShared<TILE> sh;
     const uint32_t tid = threadIdx.x;
     if (tid == 0) {
+        launch_flags() = 0;
         sh.epoch = __hip_atomic_load(&ctrl->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         sh.ntot = d_total_tiles ? *d_total_tiles : total_tiles;
     }
@@ -1765,7 +1776,10 @@ __device__ __forceinline__ void decompress_pipe_tiles(const Item it_arg, Ctrl *c
     __shared__ TileShared<TILE, C::kMaxWords> sh;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t ntot = it.ntiles;
-    if (tid == 0) sh.epoch = __hip_atomic_load(&ctrl->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) {
+        launch_flags() = 0;
+        sh.epoch = __hip_atomic_load(&ctrl->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     __syncthreads();
     const uint32_t epoch = sh.epoch;
     uint32_t ticket = 0;
@@ -1929,6 +1943,7 @@ __global__ __launch_bounds__(256) void offsets_kernel(const Item it, Ctrl *ctrl,
     const uint32_t nchunks = (it.ntiles + 63) / 64;
     const TileQ tq = {0u, 1u};   // one counter: chunks are few
     if (tid == 0) {
+        launch_flags() = 0;
         sh.epoch = __hip_atomic_load(&ctrl->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         sh.tile = tq.id(tq.take(ctrl));
     }
@@ -2386,7 +2401,8 @@ __device__ __forceinline__ void serve_consume(const SrvArgs &a, Ctrl *ctrl, uint
         uint32_t n_hdr = 0, n_words = 0;
         if (have_n) {
             if (nvalid) {
-                n_hdr = C::header(D, item_in(hb), ctrl);
+                bool rate32 = false;
+                n_hdr = C::header(D, item_in(hb), rate32);
                 n_words = header_payload_bytes(n_hdr) >> 2;
             }
             ((uint8_t *)sh.hdr[hb])[tid] = (uint8_t)n_hdr;
@@ -2466,6 +2482,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void 
 {
     __shared__ SrvShared<TILE> sh;
     if (threadIdx.x == 0) {
+        launch_flags() = 0;
         sh.t.epoch = __hip_atomic_load(&ctrl->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         sh.t.cls = __hip_atomic_fetch_add(&ctrl->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
