@@ -195,52 +195,73 @@ __device__ __forceinline__ void load_block(const Item &it, uint32_t bx, uint32_t
         // elements past z; rows whose bytes would leave the volume (its first
         // and last rows) load by elements.
         const uint16_t *vol_end = it.vol_in + (uint64_t)it.x * it.y * it.z;
-        // The common case, z odd and a wave of blocks inside the volume (not
-        // in its first or last row) whose rows have the same parities (they differ only between
-        // frames): one 16-byte load a row, from the dword boundary at or before
-        // its first element.  A row at 2 mod 4 then lacks its last element,
-        // which is the low half of the next lane's first word (v_mov_b32 with
-        // wave_shl:1): the next lane holds the next block of the row, since the
-        // block at a row's end has at most 7 elements here; only lane 63 loads
-        // it.  600 x 1813 x 1557 lossless 1.03 -> 0.77 ms and lossy 1.01 -> 0.74
+        // z odd and a wave of blocks inside the volume (all but those of its
+        // first and last rows): one 16-byte load a row, from the dword boundary
+        // at or before its first element.  A row at 2 mod 4 then lacks its last
+        // element, which is the low half of the next lane's first word
+        // (v_mov_b32 with wave_shl:1): the next lane holds the next block of the
+        // row, since the block at a row's end has at most 7 elements here; only
+        // lane 63 loads it.  Rows' parities differ between blocks only where two
+        // frames are in the wave.  600 x 1813 x 1557 lossless 1.03 -> 0.745 ms
         // against the code below, which loads the 20 bytes of such a row by two
-        // instructions and tests every row.
+        // instructions and waits for each row before the next: a workgroup is
+        // as slow as its slowest wave, so waves of two frames or with a frame's
+        // last rows are not left to it (800 x 621 x 621 dense 258 -> 214 us,
+        // 99 x 335 x 501 23.5 -> 20.9 us).
         const bool inside = p > it.vol_in && p + (uint64_t)(ny - 1u) * it.z + 9 <= vol_end;
-        const uint32_t u = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p >> 1) & 1u;
-        if (kRows == ROWS_ODD && (it.z & 1u) && __ballot(!inside || (((uint32_t)(uintptr_t)p >> 1) & 1u) != u) == 0) {
+        if (kRows == ROWS_ODD && (it.z & 1u) && __ballot(!inside) == 0) {
             uint4 t[8];
             uint32_t e[4] = {0, 0, 0, 0};
-            if (__ballot(ny != 8u) == 0) {
+            const uint32_t par = ((uint32_t)(uintptr_t)p >> 1) & 1u, u = __builtin_amdgcn_readfirstlane(par);
+            if (__ballot(ny != 8u || par != u) == 0) {
 #pragma unroll
                 for (int r = 0; r < 8; r++) t[r] = ld16_a4(p + (uint64_t)r * it.z - ((u ^ (uint32_t)r) & 1u));
                 if ((threadIdx.x & 63u) == 63u) {
 #pragma unroll
                     for (int k = 0; k < 4; k++) e[k] = p[(uint64_t)(2 * k + (u ^ 1u)) * it.z + 7];
                 }
-            } else {   // a frame's last block row is among them
 #pragma unroll
                 for (int r = 0; r < 8; r++) {
-                    t[r] = make_uint4(0, 0, 0, 0);
-                    if ((uint32_t)r < ny) {
-                        t[r] = ld16_a4(p + (uint64_t)r * it.z - ((u ^ (uint32_t)r) & 1u));
-                        if ((threadIdx.x & 63u) == 63u) e[r >> 1] = ((u ^ (uint32_t)r) & 1u) ? p[(uint64_t)r * it.z + 7] : e[r >> 1];
+                    uint32_t d0 = t[r].x, d1 = t[r].y, d2 = t[r].z, d3 = t[r].w;
+                    if ((u ^ (uint32_t)r) & 1u) {   // uniform
+                        const uint32_t next =
+                            (uint32_t)__builtin_amdgcn_update_dpp((int)e[r >> 1], (int)d0, 0x130, 0xf, 0xf, false);
+                        d0 = __builtin_amdgcn_alignbit(d1, d0, 16);
+                        d1 = __builtin_amdgcn_alignbit(d2, d1, 16);
+                        d2 = __builtin_amdgcn_alignbit(d3, d2, 16);
+                        d3 = __builtin_amdgcn_alignbit(next, d3, 16);
+                    }
+                    D[4 * r] = d0;
+                    D[4 * r + 1] = d1;
+                    D[4 * r + 2] = d2;
+                    D[4 * r + 3] = d3;
+                }
+            } else {
+                // A frame's last block row or two frames are among the blocks: the
+                // same with each lane's own parity.  Rows past the frame load its
+                // last one and are cleared.
+#pragma unroll
+                for (int r = 0; r < 8; r++) {
+                    const uint32_t row = (uint32_t)r < ny ? (uint32_t)r : ny - 1u;
+                    t[r] = ld16_a4(p + (uint64_t)row * it.z - ((par ^ row) & 1u));
+                }
+                if ((threadIdx.x & 63u) == 63u) {
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const uint32_t r = 2u * (uint32_t)k + (par ^ 1u);
+                        e[k] = p[(uint64_t)(r < ny ? r : ny - 1u) * it.z + 7];
                     }
                 }
-            }
 #pragma unroll
-            for (int r = 0; r < 8; r++) {
-                uint32_t d0 = t[r].x, d1 = t[r].y, d2 = t[r].z, d3 = t[r].w;
-                if ((u ^ (uint32_t)r) & 1u) {   // uniform
-                    const uint32_t next = (uint32_t)__builtin_amdgcn_update_dpp((int)e[r >> 1], (int)d0, 0x130, 0xf, 0xf, false);
-                    d0 = __builtin_amdgcn_alignbit(d1, d0, 16);
-                    d1 = __builtin_amdgcn_alignbit(d2, d1, 16);
-                    d2 = __builtin_amdgcn_alignbit(d3, d2, 16);
-                    d3 = __builtin_amdgcn_alignbit(next, d3, 16);
+                for (int r = 0; r < 8; r++) {
+                    const uint32_t next =
+                        (uint32_t)__builtin_amdgcn_update_dpp((int)e[r >> 1], (int)t[r].x, 0x130, 0xf, 0xf, false);
+                    const uint32_t s = 16u * ((par ^ (uint32_t)r) & 1u), m = (uint32_t)r < ny ? ~0u : 0u;
+                    D[4 * r] = __builtin_amdgcn_alignbit(t[r].y, t[r].x, s) & m;
+                    D[4 * r + 1] = __builtin_amdgcn_alignbit(t[r].z, t[r].y, s) & m;
+                    D[4 * r + 2] = __builtin_amdgcn_alignbit(t[r].w, t[r].z, s) & m;
+                    D[4 * r + 3] = __builtin_amdgcn_alignbit(next, t[r].w, s) & m;
                 }
-                D[4 * r] = d0;
-                D[4 * r + 1] = d1;
-                D[4 * r + 2] = d2;
-                D[4 * r + 3] = d3;
             }
             if (nz != 8u) {   // a block at a row end: clear the elements past z
                 const uint32_t m0 = nz > 1u ? ~0u : 0xffffu, m1 = nz > 3u ? ~0u : nz > 2u ? 0xffffu : 0u,
