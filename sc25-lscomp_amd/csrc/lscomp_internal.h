@@ -133,7 +133,10 @@ struct LaunchCfg {
     uint64_t *tile_off;              // decompress, single item: if set, tile offsets (ntiles + 1
                                      // epoch-tagged words) are computed first and the decode needs no look-back
     uint32_t off_mode;               // with tile_off: OFF_PHASE or OFF_KERNEL
+    uint32_t help;                   // compress, small volumes: probes of a missing total before a workgroup
+                                     // forms it itself, at most kHelpProbes
 };
+constexpr uint32_t kHelpProbes = 1024;
 // How a single-volume decode gets its tile offsets: a first phase of the decode
 // launch (OFF_PHASE) or a separate pre-pass kernel (OFF_KERNEL).
 enum : uint32_t { OFF_PHASE = 1, OFF_KERNEL = 2 };

@@ -21,19 +21,11 @@
 // coalesced loads (for dense streams one tile ahead), and each lane unpacks
 // its block and writes its rows.  Rate-0 blocks decode to zeros.  uint32 volumes run the same
 // kernels with the uint32 codec.
-#include <cstdlib>
 #include "lscomp_internal.h"
 
 namespace lsc {
 
 constexpr uint32_t kSpinLimit = 1u << 16;
-// Probes of a missing total before a workgroup forms it itself
-// (compress_small_tile); LSCOMP_HELP_PROBES in the environment sets another
-// number.
-static const uint32_t kHelpProbes = [] {
-    const char *e = std::getenv("LSCOMP_HELP_PROBES");
-    return e ? (uint32_t)std::strtoul(e, nullptr, 10) : 1024u;
-}();
 
 // 16 bytes at 4-byte alignment.  Volume rows and stream bytes are in general
 // only dword aligned (volumes and stream buffers at 4-byte alignment are
@@ -2066,27 +2058,27 @@ static bool use_pipe_decode(const Item &it)
 
 // Small compressions (compress_small_tile), any kind of settings.
 template <int TILE>
-static void launch_small_t(Item it, Ctrl *ctrl, uint64_t *status, hipStream_t stream)
+static void launch_small_t(Item it, uint32_t help, Ctrl *ctrl, uint64_t *status, hipStream_t stream)
 {
     it.ntiles = (it.nblocks + TILE - 1) / TILE;
     const dim3 grid(it.ntiles), block(TILE);
     if (it.dec.flags & DEC_LOSSLESS)
         hipLaunchKernelGGL((compress_small_kernel<CodecU16T<false, KIND_LOSSLESS>, TILE>), grid, block, 0, stream, it,
-                           ctrl, status, kHelpProbes);
+                           ctrl, status, help);
     else if (it.dec.flags & DEC_Q24)
         hipLaunchKernelGGL((compress_small_kernel<CodecU16T<false, KIND_Q24>, TILE>), grid, block, 0, stream, it, ctrl,
-                           status, kHelpProbes);
+                           status, help);
     else
         hipLaunchKernelGGL((compress_small_kernel<CodecU16T<false>, TILE>), grid, block, 0, stream, it, ctrl, status,
-                           kHelpProbes);
+                           help);
 }
 
 template <int TILE>
-static void launch_small_u32_t(Item it, Ctrl *ctrl, uint64_t *status, hipStream_t stream)
+static void launch_small_u32_t(Item it, uint32_t help, Ctrl *ctrl, uint64_t *status, hipStream_t stream)
 {
     it.ntiles = (it.nblocks + TILE - 1) / TILE;
     hipLaunchKernelGGL((compress_small_kernel<CodecU32, TILE>), dim3(it.ntiles), dim3(TILE), 0, stream, it, ctrl, status,
-                       kHelpProbes);
+                       help);
 }
 
 // Blocks per tile of a small compression: the smallest tile that keeps the
@@ -2121,13 +2113,13 @@ static void launch_small_decode(const Item &it, Ctrl *ctrl, hipStream_t stream)
     else launch_small_decode_t<512>(it, ctrl, stream);
 }
 
-static hipError_t launch_small(const Item &it, Ctrl *ctrl, uint64_t *status, hipStream_t stream)
+static hipError_t launch_small(const Item &it, uint32_t help, Ctrl *ctrl, uint64_t *status, hipStream_t stream)
 {
     switch (small_tile(it.nblocks)) {
-    case 64: launch_small_t<64>(it, ctrl, status, stream); break;
-    case 128: launch_small_t<128>(it, ctrl, status, stream); break;
-    case 256: launch_small_t<256>(it, ctrl, status, stream); break;
-    default: launch_small_t<512>(it, ctrl, status, stream); break;
+    case 64: launch_small_t<64>(it, help, ctrl, status, stream); break;
+    case 128: launch_small_t<128>(it, help, ctrl, status, stream); break;
+    case 256: launch_small_t<256>(it, help, ctrl, status, stream); break;
+    default: launch_small_t<512>(it, help, ctrl, status, stream); break;
     }
     return hipGetLastError();
 }
@@ -2566,9 +2558,9 @@ hipError_t launch_u32(bool compress, const Item &it, LaunchCfg cfg, Ctrl *ctrl, 
     if (cfg.tile != (uint32_t)(compress ? T : TD)) return hipErrorInvalidValue;
     const dim3 grid(cfg.grid);
     if (compress && it.ntiles <= kSmallTiles) {   // of 256 blocks
-        if (it.nblocks <= 64u * 64u) launch_small_u32_t<64>(it, ctrl, status, stream);
-        else if (it.nblocks <= 128u * 128u) launch_small_u32_t<128>(it, ctrl, status, stream);
-        else launch_small_u32_t<T>(it, ctrl, status, stream);
+        if (it.nblocks <= 64u * 64u) launch_small_u32_t<64>(it, cfg.help, ctrl, status, stream);
+        else if (it.nblocks <= 128u * 128u) launch_small_u32_t<128>(it, cfg.help, ctrl, status, stream);
+        else launch_small_u32_t<T>(it, cfg.help, ctrl, status, stream);
     } else if (compress) {
         hipLaunchKernelGGL((compress_u32_kernel<T>), grid, dim3(T), 0, stream, it, ctrl, status, cfg.sched);
     } else if (it.ntiles <= kSmallDecTiles[1]) {
@@ -2591,7 +2583,7 @@ static hipError_t launch(bool compress, const Item &single, const Item *items, c
     case 256: return launch_t<256>(compress, single, items, tile_items, cfg, ctrl, status, stream);
     case 512:
         // one small volume at the default tile (another tile asks for that launch shape)
-        if (compress && !items && single.ntiles <= kSmallTiles) return launch_small(single, ctrl, status, stream);
+        if (compress && !items && single.ntiles <= kSmallTiles) return launch_small(single, cfg.help, ctrl, status, stream);
         return launch_t<512>(compress, single, items, tile_items, cfg, ctrl, status, stream);
     case kPipeTile:   // the pipelined decode of one dense volume with the offset phase only
         if (compress || items || !cfg.tile_off || cfg.off_mode != OFF_PHASE || !dense_stream(single))
