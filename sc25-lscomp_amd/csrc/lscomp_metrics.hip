@@ -349,12 +349,15 @@ struct SsimWords {
 
 typedef const __attribute__((address_space(1))) uint8_t *GlobalBytes;
 
-// The words from the dword boundary at or before element c of each row.
+// The words from the dword boundary at or before element c0 + `at` bytes of each
+// row.  c0 is the workgroup's first element, so the lane's own offset stays
+// within a wave's words however long the rows are.
 template <bool kOdd>
 __device__ __forceinline__ void ssim_load(const uint16_t *ori, const uint16_t *dec, uint64_t plane, uint32_t Y,
-                                          uint32_t Z, uint32_t y0, uint32_t c, uint32_t odd0, SsimWords &w)
+                                          uint32_t Z, uint32_t y0, uint32_t c0, uint32_t at, uint32_t odd0, SsimWords &w)
 {
-    uint32_t at = 2u * c;
+    ori += c0;
+    dec += c0;
     asm("" : "+v"(at));   // keeps the zero extension beside the loads, which take it as their offset
 #pragma unroll
     for (uint32_t r = 0; r < kSsimRows; r++) {
@@ -418,24 +421,25 @@ __device__ __forceinline__ void ssim_plane(const SsimWords &w, SsimMom P[kSsimJ]
     P[1] = col_window(b);
 }
 
-// One workgroup per (size0 tile, size1 tile, size2 chunk) of windows; grid nb0
-// * nb1 * nchunks workgroups of 256 threads; partial[blockIdx.x] = the sum of
-// the SSIM of its windows.  odd0: bit 0 (1) is set when the original (decoded)
+// One workgroup of 256 threads per (size0 tile, size1 tile, size2 chunk) of
+// windows, nb0 * nb1 * nchunks in all, of which the launch runs those from
+// `first` on; partial[first + blockIdx.x] = the sum of the SSIM of its windows.  odd0: bit 0 (1) is set when the original (decoded)
 // volume starts at 2 mod 4.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void ssim_kernel(
     const uint16_t *__restrict__ ori, const uint16_t *__restrict__ dec, uint32_t X, uint32_t Y, uint32_t Z, uint32_t n0,
-    uint32_t n1, uint32_t n2, uint32_t nb0, uint32_t nb1, uint32_t chunk, uint32_t odd0, double *__restrict__ partial)
+    uint32_t n1, uint32_t n2, uint32_t nb0, uint32_t nb1, uint32_t chunk, uint32_t odd0, uint32_t first,
+    double *__restrict__ partial)
 {
     __shared__ double wsum[4];
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    uint32_t blk = blockIdx.x;
+    uint32_t blk = first + blockIdx.x;
     const uint32_t b0 = blk % nb0;
     blk /= nb0;
     const uint32_t b1 = blk % nb1, b2 = blk / nb1;
     const uint32_t o0 = b0 * kSsimT0 + lane, o1 = b1 * kSsimT1 + wave * kSsimJ, o2 = b2 * chunk;
     const uint32_t nw = n2 - o2 < chunk ? n2 - o2 : chunk;   // windows along size2
     // a lane's word: that of its window, and for the last windows the three words after them
-    const uint32_t c = 2u * (o0 < n0 + 2u ? o0 : n0 + 2u);
+    const uint32_t o = o0 < n0 + 2u ? o0 : n0 + 2u, c = 2u * o, c0 = 2u * (b0 * kSsimT0), at = 4u * (o - b0 * kSsimT0);
     const bool odd = (Z & 1u) || odd0;
     double acc = 0.0;
     if (o1 < n1) {
@@ -455,9 +459,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         };
         SsimWords next;
         if (odd)
-            ssim_load<true>(ori, dec, safe(plane), Y, Z, 2u * o1, c, odd0, next);
+            ssim_load<true>(ori, dec, safe(plane), Y, Z, 2u * o1, c0, at, odd0, next);
         else
-            ssim_load<false>(ori, dec, safe(plane), Y, Z, 2u * o1, c, odd0, next);
+            ssim_load<false>(ori, dec, safe(plane), Y, Z, 2u * o1, c0, at, odd0, next);
         // planes 2 o2 .. 2 o2 + 2 nw + 4, the last one at most X - 1
         for (uint32_t i = 0; i < 2u * nw + 5u; i++, plane += per_plane) {
             SsimMom P[kSsimJ];
@@ -465,9 +469,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
             if (i == 2u * nw + 4u)
                 ;
             else if (odd)
-                ssim_load<true>(ori, dec, safe(plane + per_plane), Y, Z, 2u * o1, c, odd0, next);
+                ssim_load<true>(ori, dec, safe(plane + per_plane), Y, Z, 2u * o1, c0, at, odd0, next);
             else
-                ssim_load<false>(ori, dec, safe(plane + per_plane), Y, Z, 2u * o1, c, odd0, next);
+                ssim_load<false>(ori, dec, safe(plane + per_plane), Y, Z, 2u * o1, c0, at, odd0, next);
             if ((plane == 0 && edge0) || (plane == last && edge1))
                 ssim_words_by_element(ori, dec, plane, Y, Z, 2u * o1, c, w);
             else if (odd)
@@ -504,7 +508,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o, 64);
     if (lane == 0) wsum[wave] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) partial[blockIdx.x] = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
+    if (threadIdx.x == 0) partial[first + blockIdx.x] = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
 }
 
 // The sum of np partials in a fixed order: thread t adds t, t + 1024, ...
@@ -614,8 +618,12 @@ extern "C" int lscomp_ssim_u16(const uint16_t *d_orig, const uint16_t *d_dec, ls
     if (st) return st;
     double *partial = (double *)aux.device();
     const uint32_t odd0 = (uint32_t)((uintptr_t)d_orig >> 1 & 1u) | (uint32_t)((uintptr_t)d_dec >> 1 & 1u) << 1;
-    hipLaunchKernelGGL(ssim_kernel, dim3((uint32_t)blocks), dim3(256), 0, stream, d_orig, d_dec, dims.x, dims.y,
-                       dims.z, n0, n1, n2, nb0, nb1, chunk, odd0, partial + 1);
+    // a launch holds fewer than 2^32 threads, so 2^23 workgroups each
+    for (uint64_t first = 0; first < blocks; first += 1u << 23) {
+        const uint64_t n = blocks - first < 1u << 23 ? blocks - first : 1u << 23;
+        hipLaunchKernelGGL(ssim_kernel, dim3((uint32_t)n), dim3(256), 0, stream, d_orig, d_dec, dims.x, dims.y, dims.z,
+                           n0, n1, n2, nb0, nb1, chunk, odd0, (uint32_t)first, partial + 1);
+    }
     hipLaunchKernelGGL(ssim_finish_kernel, dim3(1), dim3(1024), 0, stream, partial + 1, blocks, partial);
     st = hip_fail(hipGetLastError(), "ssim launch");
     if (!st) st = aux.read_back(sizeof(double));

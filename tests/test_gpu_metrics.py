@@ -195,3 +195,32 @@ def test_ssim_wave_edges_and_products(gpu, orc, shape):
         for x, y in ((a, b), (np.full_like(a, top - 1), b), (a, a)):
             got, want = gpu.ssim(_dev(x), _dev(y), shape), orc.ssim(x, y)
             assert got == pytest.approx(want, rel=1e-10, abs=1e-13), top
+
+
+# rows of more than 2^31 elements: 210 GB, the decoded volume the original's own
+# memory some elements on, zeros but for values in the last columns.  A window of
+# zeros has an SSIM of 1 exactly, so the sum over all windows is their number and
+# what the last columns' windows lack; sums of 2^30 terms of at most 1 in doubles
+# are good to 2^30 * 2^-53 * some tens, below 1e-5.
+@pytest.mark.parametrize("shift", [2, 1], ids=["even", "odd"])
+def test_ssim_rows_beyond_2_31(gpu, orc, shift):
+    import torch
+    z, w = (1 << 31) + 100, 164
+    n = 49 * z
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 2 * n + (2 << 30):
+        pytest.skip("needs 210 GB of free device memory")
+    rng = np.random.default_rng(shift)
+    small = np.zeros((7, 7, w), np.uint16)
+    small[:, :, w - 90:] = rng.integers(0, 4000, (7, 7, 90))
+    dec = np.zeros_like(small)
+    dec[:, :, :w - shift] = small[:, :, shift:]
+    buf = torch.zeros(n + 8, dtype=torch.int16, device="cuda")
+    buf[:n].view(7, 7, z)[:, :, z - w:].copy_(torch.from_numpy(small.view(np.int16)))
+    windows, last = (z - 7) // 2 + 1, (w - 7) // 2 + 1
+    got = gpu.ssim(buf[:n], buf[shift:n + shift], (7, 7, z))
+    del buf
+    torch.cuda.empty_cache()
+    lack = last * (1.0 - orc.ssim(small, dec))
+    assert lack > 1.0
+    assert windows * (1.0 - got) == pytest.approx(lack, abs=1e-4)
