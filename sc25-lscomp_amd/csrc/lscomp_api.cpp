@@ -420,7 +420,7 @@ int launch_item(Scratch *s, Item &it, bool compress, const Shape &shape, uint32_
     }
     LaunchCfg dcfg = cfg;
     const int mode = g_decode_mode.load();
-    if (mode == 1 && shape.tile == 512 && it.ntiles > kSmallDecTiles[0] && dense_stream(it)) {
+    if (mode == 1 && shape.tile == 512 && !small_volume(false, 512, it.ntiles) && dense_stream(it)) {
         // the pipelined decoder on tiles of kPipeTile blocks, one 16-wave workgroup
         // per CU: CSSI-shaped lossless decode 0.766 -> 0.686 ms against tiles of 512
         it.ntiles = (uint32_t)((it.nblocks + kPipeTile - 1) / kPipeTile);

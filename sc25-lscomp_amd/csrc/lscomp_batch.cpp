@@ -315,7 +315,7 @@ int lscomp_plan_autotune(lscomp_plan p, int reps, hipStream_t stream, lscomp_tun
         return rs == LSCOMP_OK ? ms : -1.0f;
     };
     Shape best{};
-    int st = tune_shape(p->direction, true, saved, measure, best, log);
+    int st = tune_shape(p->direction, true, 0, saved, measure, best, log);
     if (!st) st = apply_shape(p, best, stream);
     if (st) {
         (void)apply_shape(p, saved, stream);

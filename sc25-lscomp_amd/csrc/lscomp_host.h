@@ -33,9 +33,10 @@ int plan_take_error_async(lscomp_plan p, uint32_t *h_err, hipStream_t stream);
 // Autotuner (lscomp_tune.cpp): the average ms of `reps` calls of fn on stream
 // after one warm-up (negative if a call fails; its status in *status), and a
 // coordinate descent over the shape axes from `start` with `measure` (ms of a
-// shape, negative on failure), logging every measured shape.
+// shape, negative on failure), logging every measured shape.  `blocks`: those of
+// the single volume tuned on (0 for a plan).
 float time_launches(hipStream_t stream, int reps, const std::function<int()> &fn, int *status);
-int tune_shape(int direction, bool table, Shape start, const std::function<float(const Shape &)> &measure,
+int tune_shape(int direction, bool table, uint64_t blocks, Shape start, const std::function<float(const Shape &)> &measure,
                Shape &best, std::vector<lscomp_tune_entry> &log);
 // Grid and scheduling of a launch of `total_tiles` tiles with a normalized shape.
 LaunchCfg make_cfg(uint64_t total_tiles, bool compress, bool table, const Shape &shape);

@@ -163,6 +163,13 @@ constexpr uint32_t kTileU32 = 256;
 // one 16-wave workgroup per CU.
 constexpr uint32_t kSmallTiles = 256;
 constexpr uint32_t kSmallDecTiles[2] = {704, 448};   // uint16, uint32
+// Whether one volume of ntiles tiles of `tile` blocks (128, 256 or 512, uint16)
+// runs with one workgroup per tile.  Such a launch has no workgroups per CU,
+// counters, window or offset mode: only its tile is a choice.
+constexpr bool small_volume(bool compress, uint32_t tile, uint64_t ntiles)
+{
+    return compress ? tile == 512 && ntiles <= kSmallTiles : ntiles <= (tile == 512 ? kSmallDecTiles[0] : kSmallTiles);
+}
 constexpr uint32_t kPipeTile = 1024;
 constexpr uint32_t kTileU32Dec = 512;
 constexpr uint32_t tile_u32(bool compress) { return compress ? kTileU32 : kTileU32Dec; }

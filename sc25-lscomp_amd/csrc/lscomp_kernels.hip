@@ -2163,9 +2163,9 @@ static hipError_t launch_t(bool compress, const Item &single, const Item *items,
         else if (items)
             hipLaunchKernelGGL((decompress_kernel<TILE, true>), grid, block, 0, stream, single, items, tile_items,
                                cfg.total_tiles, cfg.d_total_tiles, ctrl, status, (uint64_t *)nullptr, sc, 0u);
-        else if (TILE == 512 && single.ntiles <= kSmallDecTiles[0])
+        else if (TILE == 512 && small_volume(false, TILE, single.ntiles))
             launch_small_decode(single, ctrl, stream);
-        else if (single.ntiles <= kSmallTiles)
+        else if (small_volume(false, TILE, single.ntiles))
             hipLaunchKernelGGL((decompress_small_kernel<TILE>), dim3(single.ntiles), block, 0, stream, single, ctrl);
         else
         {
@@ -2583,7 +2583,8 @@ static hipError_t launch(bool compress, const Item &single, const Item *items, c
     case 256: return launch_t<256>(compress, single, items, tile_items, cfg, ctrl, status, stream);
     case 512:
         // one small volume at the default tile (another tile asks for that launch shape)
-        if (compress && !items && single.ntiles <= kSmallTiles) return launch_small(single, cfg.help, ctrl, status, stream);
+        if (compress && !items && small_volume(true, 512, single.ntiles))
+            return launch_small(single, cfg.help, ctrl, status, stream);
         return launch_t<512>(compress, single, items, tile_items, cfg, ctrl, status, stream);
     case kPipeTile:   // the pipelined decode of one dense volume with the offset phase only
         if (compress || items || !cfg.tile_off || cfg.off_mode != OFF_PHASE || !dense_stream(single))

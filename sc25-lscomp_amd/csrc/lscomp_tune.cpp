@@ -6,8 +6,11 @@
 // so they are one candidate), look-back window (64 .. tile words) and tile-id
 // counters (1 .. 16).  Coordinate descent from the current shape: each axis
 // in turn, every value of it with the others held, keeping a value only when
-// it is at least 1 % faster.  Single volumes tune both directions on the
-// caller's volume (lscomp_autotune_u16, cached per size class and mode);
+// it is at least 1 % faster.  Where the launch has only a tile (small_volume) the
+// values of the other axes are measured but never kept: they are the same
+// launch, and their differences are noise.  Single volumes tune both directions
+// on the caller's volume (lscomp_autotune_u16, cached per size class, per kind of
+// launch at the default tile, and mode);
 // plans tune on their own batch (lscomp_plan_autotune, lscomp_batch.cpp).
 #include <hip/hip_runtime.h>
 
@@ -95,7 +98,7 @@ bool same_shape(const Shape &a, const Shape &b)
 
 }  // namespace
 
-int tune_shape(int direction, bool table, Shape start, const std::function<float(const Shape &)> &measure,
+int tune_shape(int direction, bool table, uint64_t blocks, Shape start, const std::function<float(const Shape &)> &measure,
                Shape &best, std::vector<lscomp_tune_entry> &log)
 {
     int st = normalize_shape(direction, start);
@@ -113,9 +116,11 @@ int tune_shape(int direction, bool table, Shape start, const std::function<float
     float best_ms = run(best);
     if (best_ms <= 0.0f) return LSCOMP_ERR_INTERNAL;
     for (int axis = 0; axis < 4; axis++) {
+        const bool same =
+            axis > 0 && !table && small_volume(direction == 0, best.tile, (blocks + best.tile - 1) / best.tile);
         for (const Shape &s : axis_values(axis, best, direction, table)) {
             const float ms = run(s);
-            if (ms > 0.0f && ms < 0.99f * best_ms) {
+            if (!same && ms > 0.0f && ms < 0.99f * best_ms) {
                 best = s;
                 best_ms = ms;
             }
@@ -133,13 +138,21 @@ struct Best {
 };
 
 std::mutex g_mu;
-std::map<std::tuple<int, int, int>, Best> g_cache;   // (device, log2 blocks, mode) -> shapes
+std::map<std::tuple<int, int, int, int>, Best> g_cache;   // (device, log2 blocks, launch_kind, mode) -> shapes
 
 int size_class(uint64_t blocks)
 {
     int c = 0;
     while ((1ull << (c + 1)) <= blocks) c++;
     return c;
+}
+
+// Whether each direction runs with one workgroup per tile at the default tile:
+// a size class has volumes on both sides of such a limit.
+int launch_kind(uint64_t blocks)
+{
+    const uint64_t tiles = (blocks + 511) / 512;
+    return (lsc::small_volume(true, 512, tiles) ? 1 : 0) + (lsc::small_volume(false, 512, tiles) ? 2 : 0);
 }
 
 int mode_of(lscomp_bins4 b, float p)
@@ -162,7 +175,8 @@ extern "C" int lscomp_autotune_u16(const uint16_t *d_in, uint8_t *d_stream, size
     if (st) return st;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return LSCOMP_ERR_HIP;
-    const auto key = std::make_tuple(dev, size_class(lscomp_num_blocks_u16(dims)), mode_of(bins, pooling_th));
+    const uint64_t blocks = lscomp_num_blocks_u16(dims);
+    const auto key = std::make_tuple(dev, size_class(blocks), launch_kind(blocks), mode_of(bins, pooling_th));
     {
         std::lock_guard<std::mutex> lk(g_mu);
         auto it = g_cache.find(key);
@@ -188,7 +202,7 @@ extern "C" int lscomp_autotune_u16(const uint16_t *d_in, uint8_t *d_stream, size
         }, &rs);
         return rs == LSCOMP_OK ? ms : -1.0f;
     };
-    st = tune_shape(0, false, saved[0], measure_c, best.s[0], log);
+    st = tune_shape(0, false, blocks, saved[0], measure_c, best.s[0], log);
     uint64_t n = 0;
     if (!st) {
         store_shape(0, best.s[0]);
@@ -206,7 +220,7 @@ extern "C" int lscomp_autotune_u16(const uint16_t *d_in, uint8_t *d_stream, size
         }, &rs);
         return rs == LSCOMP_OK ? ms : -1.0f;
     };
-    if (!st) st = tune_shape(1, false, saved[1], measure_d, best.s[1], log);
+    if (!st) st = tune_shape(1, false, blocks, saved[1], measure_d, best.s[1], log);
     (void)hipFree(d_size);
     if (st == LSCOMP_OK) st = lscomp_stream_status(stream);
     if (st != LSCOMP_OK) {
