@@ -109,7 +109,8 @@ int lscomp_decompress_u16_async(uint16_t *d_out, const uint8_t *d_in, size_t in_
                                 lscomp_dim3 dims, lscomp_bins4 bins, hipStream_t stream);
 
 /* Synchronizes `stream`, returns and clears errors raised by earlier async
- * calls on it (LSCOMP_ERR_CORRUPT / LSCOMP_ERR_INTERNAL), or LSCOMP_OK. */
+ * calls on it, replayed ones too (LSCOMP_ERR_CORRUPT / LSCOMP_ERR_RANGE /
+ * LSCOMP_ERR_INTERNAL), or LSCOMP_OK. */
 int lscomp_stream_status(hipStream_t stream);
 
 /* Pre-allocates the scratch of `stream` for volumes up to `dims` so that
@@ -123,9 +124,13 @@ void lscomp_release_all(void);
  * 1 = decompression; tile = 8x8 blocks per workgroup (128, 256 or 512;
  * 0 = the default, 512); wg_per_cu =
  * workgroups per CU (0 = occupancy limit).
- * Streams are identical for every shape; only speed changes.  No counterpart
- * in the reference (its grid is fixed, cuLSZ_entry.cu:100-101); set by the
- * autotuner or by hand. */
+ * Streams are identical for every shape; only speed changes.  Single volumes
+ * with few tiles run with one workgroup per tile, where the shape but for its
+ * tile has no effect: compression of at most 256 tiles of 512 (the workgroups
+ * then take 64 to 512 blocks each, by the volume), decompression of at most 704
+ * tiles of 512 (64 to 512 blocks each) or 256 tiles of 128 or 256.  No
+ * counterpart in the reference (its grid is fixed, cuLSZ_entry.cu:100-101); set
+ * by the autotuner or by hand. */
 int lscomp_set_launch_shape(int direction, uint32_t tile, uint32_t wg_per_cu);
 int lscomp_get_launch_shape(int direction, uint32_t *tile, uint32_t *wg_per_cu);
 
@@ -146,8 +151,11 @@ int lscomp_get_launch_shape_ex(int direction, lscomp_launch_shape *shape);
 /* How single-volume decompression finds each tile's payload offset:
  * 1 = from the header bytes in a first phase of the decode launch (default),
  * 2 = from the header bytes in a separate pre-pass kernel, 0 = a decoupled
- * look-back inside the decode kernel.  Returns the previous mode (negative
- * for an invalid mode).  Output is identical in every mode. */
+ * look-back inside the decode kernel.  Volumes decompressed with one workgroup
+ * per tile (lscomp_set_launch_shape; uint32: at most 448 tiles of 512 blocks)
+ * sum the header bytes before a tile in every mode; other uint32 volumes take
+ * mode 0 as 1.  Returns the previous mode (negative for an invalid mode).
+ * Output is identical in every mode. */
 int lscomp_set_decode_prepass(int mode);
 
 /* One measured launch shape (ms per call, averaged over the repetitions). */
@@ -163,9 +171,11 @@ typedef struct lscomp_tune_entry {
  * grid), look-back window and tile-id counters, from the current shape of
  * each direction, using d_stream (capacity >= lscomp_max_compressed_bytes_u16
  * (dims)) and d_decoded (same size as the volume) as work buffers; applies the
- * fastest shape of each direction with lscomp_set_launch_shape_ex.  Results
- * are cached per (size class, mode): a later call for the same class applies
- * the cached shapes without timing.  If table/n_table are given, the measured
+ * fastest shape of each direction with lscomp_set_launch_shape_ex.  Where a tile
+ * runs the volume with one workgroup per tile, the other axes are timed but stay
+ * as they were.  Results are cached per (size class, whether each direction runs
+ * so at the default tile, mode): a later call for the same class applies the
+ * cached shapes without timing.  If table/n_table are given, the measured
  * entries are copied there (up to *n_table; *n_table is set to the number
  * written, 0 for a cache hit).  No counterpart in the reference. */
 int lscomp_autotune_u16(const uint16_t *d_in, uint8_t *d_stream, size_t stream_capacity, uint16_t *d_decoded,
