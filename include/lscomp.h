@@ -117,7 +117,8 @@ int lscomp_stream_status(hipStream_t stream);
  * later calls on it perform no allocation (e.g. before hipGraph capture). */
 int lscomp_reserve_u16(lscomp_dim3 dims, hipStream_t stream);
 
-/* Releases every scratch area of the current device (synchronizes). */
+/* Releases every scratch area of the current device (synchronizes).  The area
+ * of a call that runs on another thread is freed when that call ends. */
 void lscomp_release_all(void);
 
 /* Launch shape of later calls (process-wide): direction 0 = compression,

@@ -12,7 +12,9 @@
 #include <cstdlib>
 #include <cstring>
 #include <atomic>
+#include <iterator>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <utility>
 
@@ -161,7 +163,8 @@ LaunchCfg make_cfg(uint64_t total_tiles, bool compress, bool table, const Shape 
 namespace {
 
 // ---------------------------------------------------------------------------
-// Scratch areas: one per (device, stream).
+// Scratch areas: one per (device, stream).  A call shares its area while it
+// runs, so lscomp_release_all on another thread leaves it to that call to free.
 // ---------------------------------------------------------------------------
 struct Scratch {
     int device = -1;
@@ -174,13 +177,28 @@ struct Scratch {
     CtrlHost *host = nullptr;      // pinned, written by the kernels
     void *aux = nullptr;           // device, kAuxKeep bytes (AuxLease), allocated at first use
     std::mutex mu;
+
+    Scratch(int dev, hipStream_t st) : device(dev), stream(st) {}
+    ~Scratch()
+    {
+        if (ctrl && host) (void)hipStreamSynchronize(stream);
+        if (status) (void)hipFree(status);
+        if (tile_off) (void)hipFree(tile_off);
+        if (ctrl) (void)hipFree(ctrl);
+        if (host) (void)hipHostFree(host);
+        if (aux) (void)hipFree(aux);
+    }
+    Scratch(const Scratch &) = delete;
+    Scratch &operator=(const Scratch &) = delete;
 };
+using ScratchRef = std::shared_ptr<Scratch>;
 static_assert(sizeof(CtrlHost::aux) >= kAuxHost, "AuxLease results");
 
 std::mutex g_mu;
-std::map<std::pair<int, hipStream_t>, Scratch *> g_scratch;
+// never destroyed: the process may end after the HIP runtime has
+auto &g_scratch = *new std::map<std::pair<int, hipStream_t>, ScratchRef>;
 
-Scratch *get_scratch(hipStream_t stream)
+ScratchRef get_scratch(hipStream_t stream)
 {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
@@ -188,23 +206,19 @@ Scratch *get_scratch(hipStream_t stream)
     auto key = std::make_pair(dev, stream);
     auto itr = g_scratch.find(key);
     if (itr != g_scratch.end()) return itr->second;
-    Scratch *s = new Scratch;
-    s->device = dev;
-    s->stream = stream;
-    if (hipMalloc((void **)&s->ctrl, sizeof(Ctrl)) != hipSuccess ||
-        hipHostMalloc((void **)&s->host, sizeof(CtrlHost), hipHostMallocDefault) != hipSuccess) {
-        if (s->ctrl) (void)hipFree(s->ctrl);
-        delete s;
+    ScratchRef s = std::make_shared<Scratch>(dev, stream);
+    if (hipMalloc((void **)&s->ctrl, sizeof(Ctrl)) != hipSuccess) {
+        s->ctrl = nullptr;
+        return nullptr;
+    }
+    if (hipHostMalloc((void **)&s->host, sizeof(CtrlHost), hipHostMallocDefault) != hipSuccess) {
+        s->host = nullptr;
         return nullptr;
     }
     std::memset((void *)s->host, 0, sizeof(CtrlHost));
     if (launch_fill_u64((uint64_t *)s->ctrl, sizeof(Ctrl) / 8, 0, stream) != hipSuccess ||
-        launch_fill_u64((uint64_t *)&s->ctrl->flags, 1, (uint64_t)(uintptr_t)s->host->flags, stream) != hipSuccess) {
-        (void)hipFree(s->ctrl);
-        (void)hipHostFree(s->host);
-        delete s;
+        launch_fill_u64((uint64_t *)&s->ctrl->flags, 1, (uint64_t)(uintptr_t)s->host->flags, stream) != hipSuccess)
         return nullptr;
-    }
     g_scratch[key] = s;
     return s;
 }
@@ -276,11 +290,12 @@ namespace lsc {
 
 AuxLease::AuxLease(hipStream_t stream, size_t bytes, size_t host_bytes) : stream_(stream)
 {
-    Scratch *s = get_scratch(stream);
+    const ScratchRef s = get_scratch(stream);
     if (!s || host_bytes > kAuxHost) {
         st_ = LSCOMP_ERR_HIP;
         return;
     }
+    keep_ = s;
     lk_ = std::unique_lock<std::mutex>(s->mu);
     host_ = s->host->aux;
     if (bytes > kAuxKeep) {
@@ -467,10 +482,10 @@ int lscomp_internal_compress_u16_async(const uint16_t *d_in, uint8_t *d_out, siz
     int st = prepare_compress(d_in, d_out, out_capacity, dims, bins, pooling_th, shape.tile, it);
     if (st) return st;
     it.result = d_out_bytes;
-    Scratch *s = get_scratch(stream);
+    const ScratchRef s = get_scratch(stream);
     if (!s) return LSCOMP_ERR_HIP;
     std::lock_guard<std::mutex> lk(s->mu);
-    return launch_item(s, it, true, shape, help_probes);
+    return launch_item(s.get(), it, true, shape, help_probes);
 }
 
 int lscomp_compress_u16_async(const uint16_t *d_in, uint8_t *d_out, size_t out_capacity, uint64_t *d_out_bytes,
@@ -489,15 +504,15 @@ int lscomp_compress_u16(const uint16_t *d_in, uint8_t *d_out, size_t out_capacit
     int st = prepare_compress(d_in, d_out, out_capacity, dims, bins, pooling_th, shape.tile, it);
     if (st == LSCOMP_ERR_CAPACITY) *out_bytes = lscomp_header_bytes_u16(dims);
     if (st) return st;
-    Scratch *s = get_scratch(stream);
+    const ScratchRef s = get_scratch(stream);
     if (!s) return LSCOMP_ERR_HIP;
     std::lock_guard<std::mutex> lk(s->mu);
-    st = launch_item(s, it, true, shape);
+    st = launch_item(s.get(), it, true, shape);
     if (st) return st;
-    st = wait_host(s);
+    st = wait_host(s.get());
     if (st) return st;
     *out_bytes = (size_t)*(volatile uint64_t *)&s->host->size;
-    st = take_errors(s);
+    st = take_errors(s.get());
     if (st) return st;
     return *out_bytes > out_capacity ? LSCOMP_ERR_CAPACITY : LSCOMP_OK;
 }
@@ -509,10 +524,10 @@ int lscomp_decompress_u16_async(uint16_t *d_out, const uint8_t *d_in, size_t in_
     Item it;
     int st = prepare_decompress(d_out, d_in, in_bytes, dims, bins, shape.tile, it);
     if (st) return st;
-    Scratch *s = get_scratch(stream);
+    const ScratchRef s = get_scratch(stream);
     if (!s) return LSCOMP_ERR_HIP;
     std::lock_guard<std::mutex> lk(s->mu);
-    return launch_item(s, it, false, shape);
+    return launch_item(s.get(), it, false, shape);
 }
 
 int lscomp_decompress_u16(uint16_t *d_out, const uint8_t *d_in, size_t in_bytes, lscomp_dim3 dims,
@@ -522,14 +537,14 @@ int lscomp_decompress_u16(uint16_t *d_out, const uint8_t *d_in, size_t in_bytes,
     Item it;
     int st = prepare_decompress(d_out, d_in, in_bytes, dims, bins, shape.tile, it);
     if (st) return st;
-    Scratch *s = get_scratch(stream);
+    const ScratchRef s = get_scratch(stream);
     if (!s) return LSCOMP_ERR_HIP;
     std::lock_guard<std::mutex> lk(s->mu);
-    st = launch_item(s, it, false, shape);
+    st = launch_item(s.get(), it, false, shape);
     if (st) return st;
-    st = wait_host(s);
+    st = wait_host(s.get());
     if (st) return st;
-    return take_errors(s);
+    return take_errors(s.get());
 }
 
 size_t lscomp_max_compressed_bytes_u32(lscomp_dim3 dims)
@@ -546,10 +561,10 @@ int lscomp_compress_u32_async(const uint32_t *d_in, uint8_t *d_out, size_t out_c
     int st = prepare_compress_u32(d_in, d_out, out_capacity, dims, bins, pooling_th, it);
     if (st) return st;
     it.result = d_out_bytes;
-    Scratch *s = get_scratch(stream);
+    const ScratchRef s = get_scratch(stream);
     if (!s) return LSCOMP_ERR_HIP;
     std::lock_guard<std::mutex> lk(s->mu);
-    return launch_item_u32(s, it, true);
+    return launch_item_u32(s.get(), it, true);
 }
 
 int lscomp_compress_u32(const uint32_t *d_in, uint8_t *d_out, size_t out_capacity, size_t *out_bytes,
@@ -560,15 +575,15 @@ int lscomp_compress_u32(const uint32_t *d_in, uint8_t *d_out, size_t out_capacit
     int st = prepare_compress_u32(d_in, d_out, out_capacity, dims, bins, pooling_th, it);
     if (st == LSCOMP_ERR_CAPACITY) *out_bytes = lscomp_header_bytes_u16(dims);
     if (st) return st;
-    Scratch *s = get_scratch(stream);
+    const ScratchRef s = get_scratch(stream);
     if (!s) return LSCOMP_ERR_HIP;
     std::lock_guard<std::mutex> lk(s->mu);
-    st = launch_item_u32(s, it, true);
+    st = launch_item_u32(s.get(), it, true);
     if (st) return st;
-    st = wait_host(s);
+    st = wait_host(s.get());
     if (st) return st;
     *out_bytes = (size_t)*(volatile uint64_t *)&s->host->size;
-    st = take_errors(s);
+    st = take_errors(s.get());
     if (st) return st;
     return *out_bytes > out_capacity ? LSCOMP_ERR_CAPACITY : LSCOMP_OK;
 }
@@ -579,10 +594,10 @@ int lscomp_decompress_u32_async(uint32_t *d_out, const uint8_t *d_in, size_t in_
     Item it;
     int st = prepare_decompress_u32(d_out, d_in, in_bytes, dims, bins, it);
     if (st) return st;
-    Scratch *s = get_scratch(stream);
+    const ScratchRef s = get_scratch(stream);
     if (!s) return LSCOMP_ERR_HIP;
     std::lock_guard<std::mutex> lk(s->mu);
-    return launch_item_u32(s, it, false);
+    return launch_item_u32(s.get(), it, false);
 }
 
 int lscomp_decompress_u32(uint32_t *d_out, const uint8_t *d_in, size_t in_bytes, lscomp_dim3 dims,
@@ -591,24 +606,24 @@ int lscomp_decompress_u32(uint32_t *d_out, const uint8_t *d_in, size_t in_bytes,
     Item it;
     int st = prepare_decompress_u32(d_out, d_in, in_bytes, dims, bins, it);
     if (st) return st;
-    Scratch *s = get_scratch(stream);
+    const ScratchRef s = get_scratch(stream);
     if (!s) return LSCOMP_ERR_HIP;
     std::lock_guard<std::mutex> lk(s->mu);
-    st = launch_item_u32(s, it, false);
+    st = launch_item_u32(s.get(), it, false);
     if (st) return st;
-    st = wait_host(s);
+    st = wait_host(s.get());
     if (st) return st;
-    return take_errors(s);
+    return take_errors(s.get());
 }
 
 int lscomp_stream_status(hipStream_t stream)
 {
-    Scratch *s = get_scratch(stream);
+    const ScratchRef s = get_scratch(stream);
     if (!s) return LSCOMP_ERR_HIP;
     std::lock_guard<std::mutex> lk(s->mu);
-    int st = wait_host(s);
+    int st = wait_host(s.get());
     if (st) return st;
-    return take_errors(s);
+    return take_errors(s.get());
 }
 
 int lscomp_reserve_u16(lscomp_dim3 dims, hipStream_t stream)
@@ -616,28 +631,22 @@ int lscomp_reserve_u16(lscomp_dim3 dims, hipStream_t stream)
     Item it;
     int st = make_item(dims, lscomp_bins4{1, 1, 1, 1}, 1.0f, it, 128);   // smallest tile: most words
     if (st) return st;
-    Scratch *s = get_scratch(stream);
+    const ScratchRef s = get_scratch(stream);
     if (!s) return LSCOMP_ERR_HIP;
     std::lock_guard<std::mutex> lk(s->mu);
-    return ensure_tiles(s, it.ntiles);
+    return ensure_tiles(s.get(), it.ntiles);
 }
 
 void lscomp_release_all(void)
 {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return;
+    std::map<std::pair<int, hipStream_t>, ScratchRef> gone;   // freed after g_mu is, by their last user
     std::lock_guard<std::mutex> lk(g_mu);
     for (auto itr = g_scratch.begin(); itr != g_scratch.end();) {
-        Scratch *s = itr->second;
-        if (s->device != dev) { ++itr; continue; }
-        (void)hipStreamSynchronize(s->stream);
-        if (s->status) (void)hipFree(s->status);
-        if (s->tile_off) (void)hipFree(s->tile_off);
-        if (s->ctrl) (void)hipFree(s->ctrl);
-        if (s->host) (void)hipHostFree(s->host);
-        if (s->aux) (void)hipFree(s->aux);
-        delete s;
-        itr = g_scratch.erase(itr);
+        const auto next = std::next(itr);
+        if (itr->second->device == dev) gone.insert(g_scratch.extract(itr));
+        itr = next;
     }
 }
 

@@ -3,6 +3,7 @@
 #pragma once
 #include <atomic>
 #include <functional>
+#include <memory>
 #include <mutex>
 #include <vector>
 #include <stdint.h>
@@ -65,6 +66,7 @@ public:
     int read_back(size_t bytes);
 
 private:
+    std::shared_ptr<void> keep_;   // the scratch area, released after its lock
     std::unique_lock<std::mutex> lk_;
     hipStream_t stream_;
     void *dev_ = nullptr, *host_ = nullptr;
