@@ -224,3 +224,27 @@ def test_ssim_rows_beyond_2_31(gpu, orc, shift):
     lack = last * (1.0 - orc.ssim(small, dec))
     assert lack > 1.0
     assert windows * (1.0 - got) == pytest.approx(lack, abs=1e-4)
+
+
+# the narrow sums (every value of a wave's plane below 2^12) at every alignment of
+# both volumes, and their limit: one value of 4095 or 4096 in the original or the
+# decoded volume only, in a corner, inside, or in a plane between, so that narrow
+# and wide planes meet in a window
+@pytest.mark.parametrize("oa,od", [(0, 0), (1, 1), (0, 1), (1, 0)])
+@pytest.mark.parametrize("shape", [(7, 7, 7), (8, 21, 133), (13, 24, 136), (9, 11, 265)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_ssim_narrow_limit(gpu, orc, shape, oa, od):
+    import torch
+    rng = np.random.default_rng(oa + 2 * od + sum(shape))
+    n = shape[0] * shape[1] * shape[2]
+    va, vb = (torch.zeros(n + 8, dtype=torch.int16, device="cuda")[o:o + n] for o in (oa, od))
+    places = [(0, 0, 0), tuple(k - 1 for k in shape), tuple(k // 2 for k in shape), (shape[0] // 2, 0, shape[2] - 1)]
+    for at in places:
+        for who, top in ((None, 0), (0, 4095), (0, 4096), (1, 4095), (1, 4096)):
+            a = rng.integers(0, 4000, shape).astype(np.uint16)
+            b = np.minimum(_noisy(a, rng, 50), 4094).astype(np.uint16)
+            if who is not None:
+                (a, b)[who][at] = top
+            va.copy_(_dev(a).view(-1))
+            vb.copy_(_dev(b).view(-1))
+            assert gpu.ssim(va, vb, shape) == pytest.approx(orc.ssim(a, b), rel=1e-10, abs=1e-13), (at, who, top)
