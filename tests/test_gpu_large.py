@@ -79,6 +79,19 @@ def test_offset_modes(gpu, orc, keep_shapes, mode, tile, shape):
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("mode", sorted(MODES))
+def test_settings(gpu, orc, mode, shape):
+    """Compression has a kernel per kind of settings."""
+    bins, p = MODES[mode]
+    vol = _case(orc, shape, 0)[0]
+    st, ref, refn = orc.compress(vol, bins, p, omp=True)
+    out, n = gpu.compress(_dev(vol), shape, bins, p)
+    assert st == 0 and n == refn and np.array_equal(out[:n].cpu().numpy(), ref)
+    dec = gpu.decompress(out, n, shape, bins)
+    assert np.array_equal(dec.cpu().numpy().view(np.uint16), orc.decompress(ref, shape, bins, omp=True)[1])
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("launch", [(128, 1, 128, 1), (256, 1, 256, 16), (512, 1, 512, 8), (512, 0, 64, 3), (512, 2, 256, 1)],
                          ids=lambda v: "-".join(map(str, v)))
 def test_launch_shapes(gpu, orc, keep_shapes, launch, shape):
