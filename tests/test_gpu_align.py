@@ -4,8 +4,8 @@ decompression's input (d_in) are placed at +0, +4, +8 and +12 bytes from a
 16-byte boundary, for uint16 and uint32 volumes, lossless and lossy, through
 the plain calls and through plans (each item at its own offset).  Streams and
 decoded volumes are byte-equal to the oracle's, and the bytes around each
-buffer are untouched (the 16-byte header stores, the offset phase's header
-reads and the payload loads all run at dword alignment there)."""
+buffer are untouched (the 16-byte header stores, the decode's header reads
+and the payload loads all run at dword alignment there)."""
 import numpy as np
 import pytest
 
@@ -17,9 +17,9 @@ OFFSETS = (0, 4, 8, 12)
 MODES = {"lossless": ((1, 1, 1, 1), 1.0), "lossy": ((3, 5, 10, 15), 0.5)}
 GUARD = 0xC3
 # several tiles (the look-back and the payload ring cross tiles), partial blocks;
-# the last has more than 256 tiles, so its decode reads the stream through the
-# offset phase and the pipelined (lossless) or sparse (lossy) decoder rather
-# than with one workgroup per tile
+# the last has more than 256 tiles, so it compresses on the persistent kernel (all
+# decode with one workgroup per tile; test_gpu_odd.py reads streams at each offset
+# through the offset phase)
 SHAPES = [(3, 77, 130), (5, 300, 264), (10, 1000, 1030)]
 
 

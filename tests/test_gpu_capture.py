@@ -9,7 +9,7 @@ from lsc_helpers import MODES, synth
 
 pytestmark = pytest.mark.gpu
 
-# 1, 64, 128 and 190 tiles of 64 to 512 blocks; 257 tiles compress on the persistent
+# 1, 64, 128 and 189 tiles of 64 to 512 blocks; 257 tiles compress on the persistent
 # kernel, 705 decompress on it
 SHAPES = [(1, 8, 60), (1, 512, 512), (4, 512, 510), (3, 1000, 1030), (1, 8, 8 * 131073), (1, 8, 8 * 360449)]
 

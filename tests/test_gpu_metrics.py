@@ -80,7 +80,7 @@ def _dev(v):
     return torch.from_numpy(np.ascontiguousarray(v).view(np.int16)).cuda()
 
 
-# one window; tiles of 64 x 4 windows along z, y and chunks of 64 along x,
+# one window; tiles of 61 x 8 windows along z, y and chunks of up to 32 along x,
 # with odd and even remainders; a shape whose windows end one short of z
 @pytest.mark.parametrize("shape", [(7, 7, 7), (9, 20, 140), (20, 33, 300), (140, 9, 9), (8, 14, 8), (11, 7, 270)],
                          ids=lambda s: "x".join(map(str, s)))
@@ -129,9 +129,10 @@ def test_ssim_identity_at_full_frame_size(gpu):
 
 
 # rows at every alignment of both volumes (odd widths alternate), the first and
-# last rows read by elements, 32- and 64-bit products (values on both sides of
-# 2^14, in the original only and in the decoded volume only), windows on both
-# sides of a wave's and a workgroup's
+# last rows read by elements, values of 14 bits with and without one of 15 in the
+# original only or the decoded volume only (the wide sums; test_ssim_narrow_limit
+# has the narrow ones and their limit), windows on both sides of a wave's and a
+# workgroup's
 @pytest.mark.parametrize("oa,od", [(0, 0), (1, 1), (0, 1), (1, 0)])
 @pytest.mark.parametrize("shape", [(7, 7, 7), (8, 21, 133), (13, 24, 136), (9, 11, 265)],
                          ids=lambda s: "x".join(map(str, s)))

@@ -179,8 +179,9 @@ def test_decode_oracle_stream(gpu, orc):
 def test_launch_shapes_give_identical_bytes(gpu, orc, tile, wg_per_cu):
     """The stream does not depend on the launch shape (tile size, persistent grid size).
     The 12 x 600 x 1558 volume (175,500 blocks) has more than 256 tiles at every
-    tile size, so it also decodes through the offset-phase launch; the smaller
-    one decodes with one workgroup per tile where it has at most 256."""
+    tile size, so it also decodes through the offset-phase launch at tiles of 128
+    and 256; at 512, up to 704 tiles decode with one workgroup per tile, as the
+    smaller one does where it has at most 256 (test_gpu_large.py goes past 704)."""
     try:
         for d in (gpu.COMPRESS, gpu.DECOMPRESS):
             gpu.set_launch_shape(d, tile, wg_per_cu)
@@ -223,7 +224,7 @@ def test_autotune_applies_a_shape_and_keeps_bytes(gpu, orc):
 def test_every_window_and_counter_count_gives_identical_bytes(gpu, orc, shape):
     """The stream does not depend on the look-back window or the number of tile-id
     counters (the 12 x 600 x 1558 volume decodes through the offset-phase launch
-    at every tile size)."""
+    at tiles of 128 and 256; test_gpu_large.py has volumes that do at 512)."""
     tile, w, win, nc = shape
     saved = [gpu.get_launch_shape_ex(k) for k in (gpu.COMPRESS, gpu.DECOMPRESS)]
     try:
@@ -285,8 +286,8 @@ def test_decode_with_and_without_prepass(gpu, orc, prepass):
     the decode launch (1) or a separate pre-pass kernel (2): same volume."""
     old = gpu.set_decode_prepass(prepass)
     try:
-        # the last two have more than 256 tiles (at most 256 decode with one
-        # workgroup per tile in every mode)
+        # all with one workgroup per tile, whatever the mode (up to 704 tiles);
+        # test_gpu_large.py has volumes where the modes differ
         for shape, kind in (((3, 300, 1558), "cssi"), ((1, 8, 9), "uniform"), ((64, 128, 128), "xpcs"),
                             ((2, 2048, 2056), "mixed"), ((12, 600, 1558), "cssi")):
             vol = synth(kind, shape, seed=31)
@@ -361,8 +362,9 @@ def test_decode_offset_chunks_beyond_the_grid(gpu, orc, mode):
                          ids=["256tiles", "257tiles", "128tiles", "1tile"])
 @pytest.mark.parametrize("mode", ["lossless", "b3-5-10-15_p0.5"])
 def test_small_volume_decode(gpu, orc, shape, mode):
-    """Volumes of at most 256 tiles decode with one workgroup per tile that sums
-    the header bytes before its tile itself; 257 tiles take the launch with the
-    offset phase.  Both sides of the limit equal the oracle's stream and decode."""
+    """Volumes of at most 704 tiles decode with one workgroup per tile that sums
+    the header bytes before its tile itself (test_gpu_small.py has both sides of
+    that limit); 257 tiles compress on the persistent kernel, 256 with one workgroup
+    per tile.  Both sides equal the oracle's stream and decode."""
     bins, p = MODES[mode]
     check_case(gpu, orc, synth("cssi", shape, seed=61 + shape[1] % 7), bins, p)

@@ -1,8 +1,9 @@
 """Small volumes (one workgroup per tile, no tile ids).  Compression: byte-equal
 to the oracle at the edges of the tile choice and of the path itself, over
-calls whose sizes go up and down on one scratch area, and with workgroups
-forming totals they find missing themselves (LSCOMP_HELP_PROBES=0: after the
-first probe)."""
+calls whose sizes go up and down on one scratch area.  Workgroups that form
+totals they find missing themselves are in test_gpu_help.py: the number of probes
+before they do is an argument there, and the environment variable that the last
+test here sets has no effect on the library."""
 import os
 import subprocess
 import sys
