@@ -541,7 +541,7 @@ def autotune(vol, dims, bins=LOSSLESS_BINS, pooling: float = 1.0, reps: int = 3,
     """Time every launch shape on this volume, apply the fastest per direction.
 
     Returns the measured table (list of dicts); empty when the shapes came from
-    the tuner's cache for this size class and mode.
+    the tuner's cache for this size class, kind of launch and mode.
     """
     import torch
     _check_volume(vol, dims)
